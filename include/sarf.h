@@ -198,15 +198,16 @@ int sarf_backproject_noalloc(sarf_ctx *ctx, const sarf_bp_desc *desc,
                              const double *f0, void *img, void *stream);
 
 /* ------------------------------------------------------------------------ */
-/* Matched-filter image formation (exact, O(K) per pixel and pulse):        */
+/* Matched-filter image formation (every sample of every pulse counts):     */
 /*   img[p] += sum_n sum_k ph[n*K + k] exp(j 4 pi f_{n,k} dR_n(p) / c),     */
 /*   f_{n,k} = f0[n] + k df[n],  dR_n(p) = |a_n - p| - R0_n,  z = 0,        */
 /* every pixel and every pulse (no swath gate).  Replaces run_mf +          */
 /* computeDifferentialRangeAndPhaseCorrectionsMF                            */
 /* (src/cpuBackProjection/cpuBackProjection.hpp:165-228) and                */
 /* matlab/mfBasic.m:66-89.  run_mf starts at pulse 2 (:218); callers that   */
-/* want that pass the pulses from index 2 on.  Range and phase steps per    */
-/* pixel and pulse in FP64; the sum over k in FP32 by Horner (K <= 8192).   */
+/* want that pass the pulses from index 2 on.  Range and phase per pixel    */
+/* and pulse in FP64; the sum over k (K <= 8192) from a per-pulse table of  */
+/* polynomials in FP32, exact to FP32 rounding (about 2e-7 of the image).   */
 /* ------------------------------------------------------------------------ */
 typedef struct {
     int Nx, Ny;       /* image size, >= 2 each */
