@@ -13,34 +13,39 @@ namespace fft {
 // cos(2 pi m / 16) for m = 0..15; sin(x) is cos(x - pi/2).
 template <int M>
 struct Tw16 {
-    static constexpr float c() {
-        constexpr float t[16] = {1.0f, 0.92387953251128674f, 0.70710678118654752f,
-                                 0.38268343236508978f, 0.0f, -0.38268343236508978f,
-                                 -0.70710678118654752f, -0.92387953251128674f, -1.0f,
-                                 -0.92387953251128674f, -0.70710678118654752f,
-                                 -0.38268343236508978f, 0.0f, 0.38268343236508978f,
-                                 0.70710678118654752f, 0.92387953251128674f};
+    static constexpr double c() {
+        constexpr double t[16] = {1.0, 0.92387953251128674, 0.70710678118654752,
+                                  0.38268343236508978, 0.0, -0.38268343236508978,
+                                  -0.70710678118654752, -0.92387953251128674, -1.0,
+                                  -0.92387953251128674, -0.70710678118654752,
+                                  -0.38268343236508978, 0.0, 0.38268343236508978,
+                                  0.70710678118654752, 0.92387953251128674};
         return t[M & 15];
     }
-    static constexpr float s() { return Tw16<(M + 12) & 15>::c(); }  // sin x = cos(x - pi/2)
+    static constexpr double s() { return Tw16<(M + 12) & 15>::c(); }  // sin x = cos(x - pi/2)
 };
 
-// d * e^{SIGN j 2 pi M / 16}, with the trivial rotations done exactly.
-template <int SIGN, int M>
-__device__ __forceinline__ float2 rot16(float2 d) {
+__device__ __forceinline__ float2 complex_of(float x, float y) { return make_float2(x, y); }
+__device__ __forceinline__ double2 complex_of(double x, double y) { return make_double2(x, y); }
+
+// d * e^{SIGN j 2 pi M / 16}, with the trivial rotations done exactly
+// (T2 = float2 or double2).
+template <int SIGN, int M, typename T2>
+__device__ __forceinline__ T2 rot16(T2 d) {
     constexpr int m = M & 15;
     if constexpr (m == 0) {
         return d;
     } else if constexpr (m == 8) {
-        return make_float2(-d.x, -d.y);
+        return complex_of(-d.x, -d.y);
     } else if constexpr (m == 4) {  // e^{SIGN j pi/2} = SIGN j
-        return SIGN > 0 ? make_float2(-d.y, d.x) : make_float2(d.y, -d.x);
+        return SIGN > 0 ? complex_of(-d.y, d.x) : complex_of(d.y, -d.x);
     } else if constexpr (m == 12) {
-        return SIGN > 0 ? make_float2(d.y, -d.x) : make_float2(-d.y, d.x);
+        return SIGN > 0 ? complex_of(d.y, -d.x) : complex_of(-d.y, d.x);
     } else {
-        constexpr float c = Tw16<m>::c();
-        constexpr float s = SIGN * Tw16<m>::s();
-        return make_float2(d.x * c - d.y * s, d.x * s + d.y * c);
+        using Re = decltype(T2{}.x);
+        constexpr Re c = (Re)Tw16<m>::c();
+        constexpr Re s = (Re)(SIGN * Tw16<m>::s());
+        return complex_of(d.x * c - d.y * s, d.x * s + d.y * c);
     }
 }
 
@@ -48,9 +53,10 @@ __device__ __forceinline__ float2 rot16(float2 d) {
 // natural-order input, bit-reversed output.
 template <int SIGN, int L, int S, int K>
 struct DifBfly {
-    static __device__ __forceinline__ void run(float2 *v) {
+    template <typename T2>
+    static __device__ __forceinline__ void run(T2 *v) {
         if constexpr (K < L / 2) {
-            float2 a = v[S + K], b = v[S + K + L / 2];
+            T2 a = v[S + K], b = v[S + K + L / 2];
             v[S + K] = cadd(a, b);
             v[S + K + L / 2] = rot16<SIGN, (K * 16 / L)>(csub(a, b));
             DifBfly<SIGN, L, S, K + 1>::run(v);
@@ -59,7 +65,8 @@ struct DifBfly {
 };
 template <int SIGN, int R, int L, int S>
 struct DifStage {
-    static __device__ __forceinline__ void run(float2 *v) {
+    template <typename T2>
+    static __device__ __forceinline__ void run(T2 *v) {
         if constexpr (S < R) {
             DifBfly<SIGN, L, S, 0>::run(v);
             DifStage<SIGN, R, L, S + L>::run(v);
@@ -68,7 +75,8 @@ struct DifStage {
 };
 template <int SIGN, int R, int L>
 struct DifAll {
-    static __device__ __forceinline__ void run(float2 *v) {
+    template <typename T2>
+    static __device__ __forceinline__ void run(T2 *v) {
         if constexpr (L >= 2) {
             DifStage<SIGN, R, L, 0>::run(v);
             DifAll<SIGN, R, L / 2>::run(v);
@@ -86,10 +94,10 @@ __host__ __device__ constexpr int bitrev(int x) {
 }
 
 // In-place R-point DFT (sign SIGN) of v[0..R-1], result in natural order.
-template <int SIGN, int R>
-__device__ __forceinline__ void dft(float2 *v) {
+template <int SIGN, int R, typename T2>
+__device__ __forceinline__ void dft(T2 *v) {
     DifAll<SIGN, R, R>::run(v);
-    float2 t[R];
+    T2 t[R];
 #pragma unroll
     for (int i = 0; i < R; i++) t[i] = v[bitrev<R>(i)];
 #pragma unroll
@@ -107,6 +115,25 @@ __device__ __forceinline__ void powers16_rev(float rev, float2 *p) {
         const float a = rev * (float)r;
         p[r] = make_float2(__builtin_amdgcn_cosf(a), __builtin_amdgcn_sinf(a));
     }
+}
+
+// e^{j 2 pi t}, 0 <= t <= 1, within an ulp or so of FP32 (the sine/cosine unit's
+// absolute error is about four times that): t - q/4 in [-1/8, 1/8] exactly, the
+// Taylor polynomials of sin(2 pi x) and cos(2 pi x) there (the first terms left
+// out are below 3e-9), and a quarter turn's exchange and signs.
+__device__ __forceinline__ float2 cis_rev(float t) {
+    const float q = rintf(4.f * t);
+    const float x = fmaf(-0.25f, q, t), z = x * x;
+    const float s = x * fmaf(z, fmaf(z, fmaf(z, fmaf(z, 42.058693944897658f, -76.705859753061383f),
+                                              81.605249276075054f), -41.341702240399755f),
+                             6.2831853071795865f);
+    const float c = fmaf(z, fmaf(z, fmaf(z, fmaf(z, fmaf(z, -26.426256783374398f,
+                                                         60.244641371876663f), -85.456817206693725f),
+                                         64.939394022668291f), -19.739208802178717f), 1.f);
+    const int k = (int)q;
+    const float a = (k & 1) ? s : c, b = (k & 1) ? c : s;  // |cos|, |sin| after the turns
+    // turns 0..4: (c, s), (-s, c), (-c, -s), (s, -c), (c, s)
+    return make_float2(((k + 1) & 2) ? -a : a, (k & 2) ? -b : b);
 }
 
 // w^r for r = 0..15 from w (r = 0 unused); error <= ~4 roundings.

@@ -249,156 +249,207 @@ __global__ __launch_bounds__(rc_threads(LOG2N)) void rc_lds_f32_jobs(
 }
 
 // ---------------------------------------------------------------------------
-// Global-memory Stockham, radix 4 (one radix-2 pass if log2 N is odd): the
-// FP64 path, and FP32 transforms longer than the 16384 bins that fit in
-// LDS.  Pass 0 reads the phase history (zero padding, taper, fftshift fold);
-// the last pass applies 1/N and the ramp.
+// Transforms through global memory: the FP64 path, FP32 powers of two outside
+// the 32..16384 that one workgroup holds in LDS, and the Bluestein transforms
+// beyond the register-resident ones.  Self-sorting Stockham passes of radix
+// R = 2^LOG2R <= 256 (two passes up to 2^16, three up to 2^24).  With Ns the
+// product of the earlier passes' radices, column j < N/R of a pulse is
+//   out[(j - k) R + k + r Ns] = DFT_R over r' of in[j + r' N/R] w^{r' k N/(Ns R)},
+//   k = j mod Ns,  w = e^{+j 2 pi / N}.
+// A workgroup takes C consecutive columns, 16 values per thread, so global
+// accesses are segments of C elements (128 bytes at R = 256): a thread holds
+// the elements a + R1 b, b < 16, of a column (R1 = R / 16), transforms them,
+// exchanges through LDS and finishes with radix R1.
+// Bound by memory: a radix-4 pass per factor of 4, the former form, moved every
+// bin eight times at N = 2^16 (512 x 6000 -> 65536: 1110 us, 176 now, 293 MB of
+// samples and profiles; FP64 512 x 424 -> 4096: 80 -> 43 us traced).
+// Bluestein's identity, per pulse in rows of M (see rc_bluestein below):
+//   z_k = conj(x_k taper_k c_k) for k < K, 0 up to M        (load of pass 0)
+//   Z = IFFT_M(z) unscaled = conj(FFT_M(x c))               (passes)
+//   U = conj(Z) .* C,  C = FFT_M(h), h circularly conj(c)   (store of the last)
+//   W = IFFT_M(U) unscaled = M ((x c) * h)                  (passes)
+//   X_m = c_m W_m / (M N) (ramp), at the fftshift position  (store of the last)
 // ---------------------------------------------------------------------------
-template <typename T2, int R>
-__global__ __launch_bounds__(256) void rc_pass(
-    const T2 *__restrict__ in, T2 *__restrict__ out, int N, int Ns, int Np,
-    const T2 *__restrict__ tw, int first, int K, int flags,
-    const float *__restrict__ taper, int last, const double *__restrict__ f0,
-    const double *__restrict__ r0) {
-    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long per = N / R;
-    const long n = gid / per;
-    const int j = (int)(gid % per);
-    if (n >= Np) return;
+enum : int { kLoadRows, kLoadSamples, kLoadChirped };
+enum : int { kStoreRows, kStoreProfile, kStoreSpectrum, kStoreChirped };
+
+template <typename T2>
+struct PassArgs {
+    const T2 *in;
+    T2 *out;
+    const T2 *twN;  // e^{+j 2 pi i / N}, i < N (FP64 only)
+    const T2 *twR;  // e^{+j 2 pi i / R}, i < R
+    const T2 *chirp, *C;
+    const float *taper;
+    const double *f0, *r0;
+    long cols;  // columns of all pulses
+    int log2n, log2ns;
+    int load, store;
+    int K, flags, nout;  // samples, SARF_RC_*, profile bins (kStoreChirped)
+};
+
+template <typename T2>
+constexpr int pass_threads() {
+    return sizeof(T2) == sizeof(double2) ? 128 : 256;
+}
+
+// PAST: kStoreProfile stores past the caches.
+template <typename T2, int LOG2R, bool PAST>
+__global__ __launch_bounds__(pass_threads<T2>()) void rc_pass(PassArgs<T2> p) {
     using Re = decltype(T2{}.x);
-    T2 v[R];
+    constexpr int TPB = pass_threads<T2>();
+    constexpr int R = 1 << LOG2R;
+    constexpr int RA = R < 16 ? R : 16;  // radix of the first step
+    constexpr int R1 = R / RA;           // of the second
+    constexpr int NC = 16 / RA;          // columns per thread in the first step
+    constexpr int C = TPB * 16 / R;      // columns per workgroup
+    constexpr int CP = C + 1;            // padded, columns fastest
+    __shared__ T2 xch[R1 > 1 ? R * CP : 1];
+    __shared__ T2 wR[R1 > 1 ? R : 1];
+    __shared__ double2 ramp[C];
+    const int tid = threadIdx.x;
+    const long col0 = (long)blockIdx.x * C;
+    const int log2per = p.log2n - LOG2R;
+    const long per = 1L << log2per;
+    const long N = 1L << p.log2n;
+    const int Ns = 1 << p.log2ns;
+    if (R1 > 1)
+        for (int i = tid; i < R; i += TPB) wR[i] = p.twR[i];
+    if (p.store == kStoreProfile || p.store == kStoreChirped) {
+        // scale and ramp, once per column
+        for (int c = tid; c < C; c += TPB) {
+            const double sc = p.store == kStoreProfile ? 1.0 / N : 1.0 / ((double)N * p.nout);
+            double2 f = make_double2(sc, 0.0);
+            if ((p.flags & SARF_RC_RAMP) && col0 + c < p.cols) {
+                const long n = (col0 + c) >> log2per;
+                const double a = -4.0 * kPi * p.f0[n] * p.r0[n] / kClight;
+                f = make_double2(cos(a) * sc, sin(a) * sc);
+            }
+            ramp[c] = f;
+        }
+    }
+    if (R1 > 1 || p.store == kStoreProfile || p.store == kStoreChirped) __syncthreads();
+
+    auto store = [&](int c, int r, T2 x) {
+        const long col = col0 + c;
+        if (col >= p.cols) return;
+        const long n = col >> log2per;
+        const int j = (int)(col & (per - 1)), k = j & (Ns - 1);
+        const long o = (((long)(j - k)) << LOG2R) + k + ((long)r << p.log2ns);
+        if (p.store == kStoreRows) {
+            p.out[(n << p.log2n) + o] = x;
+        } else if (p.store == kStoreProfile) {
+            const Re sr = (Re)ramp[c].x, si = (Re)ramp[c].y;
+            using V = Re __attribute__((ext_vector_type(2)));
+            const V y = {x.x * sr - x.y * si, x.x * si + x.y * sr};
+            V *dst = (V *)(p.out + (n << p.log2n) + o);
+            if constexpr (PAST) __builtin_nontemporal_store(y, dst);
+            else *dst = y;
+        } else if (p.store == kStoreSpectrum) {
+            x.y = -x.y;
+            p.out[(n << p.log2n) + o] = cmul(x, p.C[o]);
+        } else if (o < p.nout) {
+            const Re sr = (Re)ramp[c].x, si = (Re)ramp[c].y;
+            x = cmul(x, p.chirp[o]);
+            long q = o - (p.nout + 1) / 2;
+            if (q < 0) q += p.nout;
+            p.out[n * p.nout + q] = fft::complex_of(x.x * sr - x.y * si, x.x * si + x.y * sr);
+        }
+    };
+
+    // ---- load, twiddles of the earlier passes, first step -----------------
+    // lanes run along the columns; thread (c, a) holds elements a + R1 b
+    const int c = tid % C, a = R1 > 1 ? tid / C : 0;
+    T2 v[16];
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int idx = j + r * (N / R);
-        if (first) {
+    for (int i = 0; i < NC; i++) {
+        const int ci = NC > 1 ? tid + i * TPB : c;  // NC > 1: R1 = 1, one thread per column
+        const long col = col0 + ci;
+        const bool ok = col < p.cols;
+        const long n = ok ? col >> log2per : 0;
+        const int j = (int)(col & (per - 1)), k = j & (Ns - 1);
+        T2 *w = v + i * RA;
+#pragma unroll
+        for (int b = 0; b < RA; b++) {
+            const long idx = j + ((long)(a + R1 * b) << log2per);
             T2 x{};
-            if (idx < K) {
-                x = in[n * K + idx];
-                if (flags & SARF_RC_TAPER) {
-                    x.x *= taper[idx];
-                    x.y *= taper[idx];
+            if (p.load == kLoadRows) {
+                if (ok) x = p.in[(n << p.log2n) + idx];
+            } else if (ok && idx < p.K) {
+                x = p.in[n * p.K + idx];
+                if (p.flags & SARF_RC_TAPER) {
+                    x.x *= p.taper[idx];
+                    x.y *= p.taper[idx];
                 }
-                if (idx & 1) {
+                if (p.load == kLoadChirped) {
+                    x = cmul(x, p.chirp[idx]);
+                    x.y = -x.y;
+                } else if (idx & 1) {  // fftshift fold
                     x.x = -x.x;
                     x.y = -x.y;
                 }
             }
-            v[r] = x;
-        } else {
-            v[r] = in[n * N + idx];
+            w[b] = x;
         }
-    }
-    const int k = j % Ns;
+        if (Ns > 1) {
+            if constexpr (sizeof(T2) == sizeof(float2)) {
+                // r k < R Ns <= 2^24: the revolutions are exact
+                const float rev = __builtin_ldexpf((float)k, -(LOG2R + p.log2ns));
 #pragma unroll
-    for (int r = 1; r < R; r++) {
-        const long ti = (long)r * k * (N / (Ns * R));
-        v[r] = cmul(v[r], tw[ti]);
-    }
-    // inverse DFT of size R (R = 2 or 4)
-    if constexpr (R == 2) {
-        T2 a = v[0], b = v[1];
-        v[0] = cadd(a, b);
-        v[1] = csub(a, b);
-    } else {
-        T2 a0 = cadd(v[0], v[2]), a1 = csub(v[0], v[2]);
-        T2 b0 = cadd(v[1], v[3]), b1 = csub(v[1], v[3]);
-        T2 jb1;  // +j * b1
-        jb1.x = -b1.y;
-        jb1.y = b1.x;
-        v[0] = cadd(a0, b0);
-        v[2] = csub(a0, b0);
-        v[1] = cadd(a1, jb1);
-        v[3] = csub(a1, jb1);
-    }
-    double sr = 1.0, si = 0.0;
-    if (last) {
-        sr = 1.0 / N;
-        if (flags & SARF_RC_RAMP) {
-            const double a = -4.0 * kPi * f0[n] * r0[n] / kClight;
-            sr = cos(a) / N;
-            si = sin(a) / N;
-        }
-    }
-    const int base = (j - k) * R + k;
+                for (int b = 0; b < RA; b++) {
+                    w[b] = cmul(w[b], fft::cis_rev(__builtin_amdgcn_fractf(
+                                          rev * (float)(a + R1 * b))));
+                }
+            } else {
+                // w^{(a + R1 b) k s}: table entries for a and for b = 1, 2, 4,
+                // 8, the others products of at most four
+                const long s = (long)k << (p.log2n - LOG2R - p.log2ns);
+                T2 g[16];
+                g[0] = p.twN[a * s];
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        T2 x = v[r];
-        if (last) {
-            const Re xr = x.x, xi = x.y;
-            x.x = xr * (Re)sr - xi * (Re)si;
-            x.y = xr * (Re)si + xi * (Re)sr;
+                for (int b = 1; b < RA; b *= 2) {
+                    const T2 e = p.twN[(long)R1 * b * s & (N - 1)];
+#pragma unroll
+                    for (int q = 0; q < b; q++) g[b + q] = cmul(g[q], e);
+                }
+#pragma unroll
+                for (int b = 0; b < RA; b++) w[b] = cmul(w[b], g[b]);
+            }
         }
-        out[n * N + base + r * Ns] = x;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Nfft not a power of two beyond the register-resident range (FP32 above
-// 8192, every FP64 length): the same Bluestein identity as rc_bluestein below,
-// with the two length-M transforms done by the global-memory passes.  Per
-// pulse, in rows of M:
-//   rcb_pre : z_k = conj(x_k taper_k c_k) for k < K, 0 up to M
-//   passes  : Z = IFFT_M(z) unscaled = conj(FFT_M(x c))
-//   rcb_mul : U = conj(Z) .* C                         (C = FFT_M(h), h the
-//             circularly extended conj(c); FFT_M(x c) .* C = FFT_M((x c) * h))
-//   passes  : W = IFFT_M(U) unscaled = M ((x c) * h)
-//   rcb_post: X_m = c_m W_m / (M N) (ramp), stored at the fftshift position.
-// ---------------------------------------------------------------------------
-template <typename T2>
-__global__ __launch_bounds__(256) void rcb_pre(const T2 *__restrict__ ph, int K, int M, long total,
-                                               int flags, const float *__restrict__ taper,
-                                               const T2 *__restrict__ chirp, T2 *__restrict__ z) {
-    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= total) return;
-    const long n = gid / M;
-    const int k = (int)(gid - n * M);
-    T2 v{};
-    if (k < K) {
-        T2 x = ph[n * K + k];
-        if (flags & SARF_RC_TAPER) {
-            x.x *= taper[k];
-            x.y *= taper[k];
+        fft::dft<+1, RA>(w);
+        if (R1 == 1) {
+#pragma unroll
+            for (int r = 0; r < RA; r++) store(ci, r, w[r]);
         }
-        v = cmul(x, chirp[k]);
-        v.y = -v.y;
     }
-    z[gid] = v;
-}
-
-template <typename T2>
-__global__ __launch_bounds__(256) void rcb_mul(T2 *__restrict__ z, int M, long total,
-                                               const T2 *__restrict__ C) {
-    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= total) return;
-    T2 v = z[gid];
-    v.y = -v.y;
-    z[gid] = cmul(v, C[gid % M]);
-}
-
-template <typename T2>
-__global__ __launch_bounds__(256) void rcb_post(const T2 *__restrict__ w, int M, int N, long total,
-                                                int flags, const double *__restrict__ f0,
-                                                const double *__restrict__ r0,
-                                                const T2 *__restrict__ chirp, T2 *__restrict__ prof) {
-    using Re = decltype(T2{}.x);
-    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= total) return;
-    const long n = gid / N;
-    const int m = (int)(gid - n * N);
-    double sr = 1.0 / ((double)M * N), si = 0.0;
-    if (flags & SARF_RC_RAMP) {
-        const double a = -4.0 * kPi * f0[n] * r0[n] / kClight;
-        sr = cos(a) / ((double)M * N);
-        si = sin(a) / ((double)M * N);
+    if constexpr (R1 > 1) {
+        // ---- exchange: element (a, q) of column c at (a 16 + q) CP + c --------
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            T2 x = v[q];
+            if (q > 0) x = cmul(x, wR[a * q]);
+            xch[(a * 16 + q) * CP + c] = x;
+        }
+        __syncthreads();
+        // Second step: thread (c2, g) finishes outputs q + 16 p, p < R1, of the
+        // 16 / R1 values q = g 16 / R1 + i.  Lanes run along the columns where
+        // those are adjacent in the output (Ns >= C), along q in pass 0.
+        const bool along = p.log2ns > 0;
+        const int c2 = along ? tid % C : tid / R1, g = along ? tid / C : tid % R1;
+        constexpr int NQ = 16 / R1;
+#pragma unroll
+        for (int i = 0; i < NQ; i++) {
+            const int q = g * NQ + i;
+            T2 *w = v + i * R1;
+#pragma unroll
+            for (int e = 0; e < R1; e++) w[e] = xch[(e * 16 + q) * CP + c2];
+            fft::dft<+1, R1>(w);
+        }
+#pragma unroll
+        for (int e = 0; e < R1; e++)
+#pragma unroll
+            for (int i = 0; i < NQ; i++) store(c2, g * NQ + i + 16 * e, v[i * R1 + e]);
     }
-    const T2 X = cmul(w[n * M + m], chirp[m]);
-    const int half = (N + 1) / 2;
-    int o = m - half;
-    if (o < 0) o += N;
-    T2 y;
-    y.x = X.x * (Re)sr - X.y * (Re)si;
-    y.y = X.x * (Re)si + X.y * (Re)sr;
-    prof[n * N + o] = y;
 }
 
 // ---------------------------------------------------------------------------
@@ -652,88 +703,141 @@ void launch_bluestein_t(const sarf_rc_desc *d, const float2 *ph, const float *ta
                        taper, f0, r0, chirp, C, tw, prof);
 }
 
-// Stockham passes of length N = 2^log2n through global memory (ping-pong
-// with `tmp` so the last pass lands in prof).
 template <typename T2>
-int launch_passes(const sarf_rc_desc *d, int log2n, const T2 *ph, const float *taper,
-                  const double *f0, const double *r0, const T2 *tw, T2 *prof, T2 *tmp,
-                  hipStream_t s) {
-    const int npass = (log2n & 1) + log2n / 2;
-    T2 *bufs[2] = {prof, tmp};
-    int cur = (npass % 2 == 1) ? 0 : 1;  // output buffer index of pass 0
-    const T2 *in = ph;
-    int Ns = 1, pass = 0;
-    if (log2n & 1) {
-        const long threads = (long)d->Np * (d->Nfft / 2);
-        hipLaunchKernelGGL((rc_pass<T2, 2>), dim3((threads + 255) / 256), dim3(256), 0, s, in,
-                           bufs[cur], d->Nfft, Ns, d->Np, tw, 1, d->K, d->flags, taper,
-                           npass == 1, f0, r0);
-        SARF_HIP(hipGetLastError());
-        in = bufs[cur];
-        cur ^= 1;
-        Ns *= 2;
-        pass++;
+int pass_twiddles_of(sarf_ctx *ctx, int log2n, const T2 **out) {
+    if constexpr (sizeof(T2) == sizeof(double2)) return twiddles_f64(ctx, log2n, out);
+    else return twiddles_f32(ctx, log2n, out);
+}
+
+template <typename T2, int LOG2R>
+void launch_pass_t(PassArgs<T2> p, bool past, long pulses, hipStream_t s) {
+    constexpr int C = pass_threads<T2>() * 16 >> LOG2R;
+    p.cols = pulses << (p.log2n - LOG2R);
+    const dim3 grid((unsigned)((p.cols + C - 1) / C)), block(pass_threads<T2>());
+    if (past && LOG2R > 4)
+        hipLaunchKernelGGL((rc_pass<T2, LOG2R, (LOG2R > 4)>), grid, block, 0, s, p);
+    else
+        hipLaunchKernelGGL((rc_pass<T2, LOG2R, false>), grid, block, 0, s, p);
+}
+
+template <typename T2>
+void launch_pass(const PassArgs<T2> &p, int log2r, bool past, long pulses, hipStream_t s) {
+    switch (log2r) {
+        case 1: launch_pass_t<T2, 1>(p, past, pulses, s); break;
+        case 2: launch_pass_t<T2, 2>(p, past, pulses, s); break;
+        case 3: launch_pass_t<T2, 3>(p, past, pulses, s); break;
+        case 4: launch_pass_t<T2, 4>(p, past, pulses, s); break;
+        case 5: launch_pass_t<T2, 5>(p, past, pulses, s); break;
+        case 6: launch_pass_t<T2, 6>(p, past, pulses, s); break;
+        case 7: launch_pass_t<T2, 7>(p, past, pulses, s); break;
+        default: launch_pass_t<T2, 8>(p, past, pulses, s); break;
     }
-    for (; pass < npass; pass++) {
-        const long threads = (long)d->Np * (d->Nfft / 4);
-        hipLaunchKernelGGL((rc_pass<T2, 4>), dim3((threads + 255) / 256), dim3(256), 0, s, in,
-                           bufs[cur], d->Nfft, Ns, d->Np, tw, pass == 0, d->K, d->flags, taper,
-                           pass == npass - 1, f0, r0);
+}
+
+// The passes of `pulses` inverse transforms of length 2^log2n (>= 2): p gives
+// the first pass's input and load, the last one's store and output; in between
+// the rows go through x and y in turn (y unused up to two passes, both up to
+// one; past: store the profiles past the caches).  The radices' logarithms differ by at most one, the larger ones first.
+template <typename T2>
+int launch_passes(sarf_ctx *ctx, PassArgs<T2> p, int log2n, long pulses, T2 *x, T2 *y,
+                  bool past, hipStream_t s) {
+    const int npass = (log2n + 7) / 8;
+    const int load = p.load, store = p.store;
+    T2 *const last = p.out;
+    p.log2n = log2n;
+    p.log2ns = 0;
+    if (sizeof(T2) == sizeof(double2)) SARF_TRY(pass_twiddles_of(ctx, log2n, &p.twN));
+    for (int i = 0; i < npass; i++) {
+        const int l = log2n / npass + (i < log2n % npass);
+        SARF_TRY(pass_twiddles_of(ctx, l, &p.twR));
+        p.load = i == 0 ? load : (int)kLoadRows;
+        p.store = i == npass - 1 ? store : (int)kStoreRows;
+        p.out = i == npass - 1 ? last : (i & 1) ? y : x;
+        launch_pass(p, l, past && i == npass - 1, pulses, s);
         SARF_HIP(hipGetLastError());
-        in = bufs[cur];
-        cur ^= 1;
-        Ns *= 4;
+        p.in = p.out;
+        p.log2ns += l;
     }
     return SARF_OK;
 }
 
-// Unscaled inverse transforms of length M = 2^L of Np rows held in x,
-// ping-ponging with y; returns the buffer holding the result.
-template <typename T2>
-T2 *inverse_passes(T2 *x, T2 *y, int L, int Np, const T2 *tw, hipStream_t s) {
-    const int M = 1 << L;
-    T2 *in = x, *out = y;
-    int Ns = 1;
-    if (L & 1) {
-        const long threads = (long)Np * (M / 2);
-        hipLaunchKernelGGL((rc_pass<T2, 2>), dim3((threads + 255) / 256), dim3(256), 0, s, in, out,
-                           M, Ns, Np, tw, 0, M, 0, nullptr, 0, nullptr, nullptr);
-        std::swap(in, out);
-        Ns *= 2;
-    }
-    for (; Ns < M; Ns *= 4) {
-        const long threads = (long)Np * (M / 4);
-        hipLaunchKernelGGL((rc_pass<T2, 4>), dim3((threads + 255) / 256), dim3(256), 0, s, in, out,
-                           M, Ns, Np, tw, 0, M, 0, nullptr, 0, nullptr, nullptr);
-        std::swap(in, out);
-    }
-    return in;
+// Pulses per slab: the passes of a slab follow each other before the next
+// slab's, so the rows between them stay in the 256 MB last-level cache (and the
+// scratch small).  512 x 6000 -> 65536: slabs of 32 MB 308 us, 64 MB 234, 128 MB
+// 208, 256 MB and more 252.  Profiles that would fill that cache themselves
+// are stored past it: 176 us.
+constexpr size_t kSlabBytes = size_t(128) << 20;
+int pulses_per_slab(size_t row_bytes, int Np) {
+    return (int)std::min<long>(Np, std::max<long>(1, (long)(kSlabBytes / row_bytes)));
 }
 
-// Bluestein through global memory (rcb_pre / passes / rcb_mul / passes /
-// rcb_post), two scratch rows of M per pulse.
+// Range compression of length 2^log2n through the passes.
+template <typename T2>
+int launch_long(sarf_ctx *ctx, const sarf_rc_desc *d, int log2n, const T2 *ph,
+                const float *taper, const double *f0, const double *r0, T2 *prof, hipStream_t s) {
+    const size_t row = sizeof(T2) << log2n;
+    const int npass = (log2n + 7) / 8, slab = pulses_per_slab(row, d->Np);
+    const bool past = row * d->Np > kSlabBytes;
+    const char *name = sizeof(T2) == sizeof(double2) ? "rc64.tmp" : "rc32.tmp";
+    T2 *x = nullptr, *y = nullptr;
+    if (npass > 1) {
+        void *b = nullptr;
+        SARF_TRY(scratch_get(ctx, name, row * slab * (npass - 1), &b));
+        x = (T2 *)b;
+        y = x + ((size_t)slab << log2n);
+    }
+    for (int n0 = 0; n0 < d->Np; n0 += slab) {
+        PassArgs<T2> p{};
+        p.in = ph + (size_t)n0 * d->K;
+        p.out = prof + ((size_t)n0 << log2n);
+        p.load = kLoadSamples;
+        p.store = kStoreProfile;
+        p.K = d->K;
+        p.flags = d->flags;
+        p.taper = taper;
+        p.f0 = f0 ? f0 + n0 : nullptr;
+        p.r0 = r0 ? r0 + n0 : nullptr;
+        SARF_TRY(launch_passes(ctx, p, log2n, std::min(slab, d->Np - n0), x, y, past, s));
+    }
+    return SARF_OK;
+}
+
+// Bluestein through the passes: scratch rows of M = 2^L, two per pulse (three
+// when a transform takes three passes).
 template <typename T2>
 int launch_bluestein_global(sarf_ctx *ctx, const sarf_rc_desc *d, int L, const T2 *ph,
-                            const float *taper, const double *f0, const double *r0,
-                            const T2 *tw, T2 *prof, hipStream_t s) {
-    const int N = d->Nfft, M = 1 << L;
+                            const float *taper, const double *f0, const double *r0, T2 *prof,
+                            hipStream_t s) {
+    const int N = d->Nfft;
     const T2 *chirp = nullptr, *C = nullptr;
     SARF_TRY(bluestein_tables<T2>(ctx, N, L, &chirp, &C));
-    const long rows = (long)d->Np * M;
-    void *a = nullptr, *b = nullptr;
-    SARF_TRY(scratch_get(ctx, "rcb.a", sizeof(T2) * (size_t)rows, &a));
-    SARF_TRY(scratch_get(ctx, "rcb.b", sizeof(T2) * (size_t)rows, &b));
-    T2 *za = (T2 *)a, *zb = (T2 *)b;
-    const dim3 gm((unsigned)((rows + 255) / 256));
-    hipLaunchKernelGGL(rcb_pre<T2>, gm, dim3(256), 0, s, ph, d->K, M, rows, d->flags, taper,
-                       chirp, za);
-    T2 *z = inverse_passes<T2>(za, zb, L, d->Np, tw, s);
-    hipLaunchKernelGGL(rcb_mul<T2>, gm, dim3(256), 0, s, z, M, rows, C);
-    T2 *w = inverse_passes<T2>(z, z == za ? zb : za, L, d->Np, tw, s);
-    const long outs = (long)d->Np * N;
-    hipLaunchKernelGGL(rcb_post<T2>, dim3((unsigned)((outs + 255) / 256)), dim3(256), 0, s, w, M, N,
-                       outs, d->flags, f0, r0, chirp, prof);
-    SARF_HIP(hipGetLastError());
+    const size_t row = sizeof(T2) << L;
+    const int npass = (L + 7) / 8, slab = pulses_per_slab(row, d->Np);
+    void *b = nullptr;
+    SARF_TRY(scratch_get(ctx, "rcb.rows", row * slab * std::max(2, npass), &b));
+    T2 *u = (T2 *)b, *x = u + ((size_t)slab << L), *y = x + ((size_t)slab << L);
+    for (int n0 = 0; n0 < d->Np; n0 += slab) {
+        const int np = std::min(slab, d->Np - n0);
+        PassArgs<T2> p{};
+        p.in = ph + (size_t)n0 * d->K;
+        p.out = u;
+        p.load = kLoadChirped;
+        p.store = kStoreSpectrum;
+        p.K = d->K;
+        p.flags = d->flags;
+        p.nout = N;
+        p.taper = taper;
+        p.chirp = chirp;
+        p.C = C;
+        p.f0 = f0 ? f0 + n0 : nullptr;
+        p.r0 = r0 ? r0 + n0 : nullptr;
+        SARF_TRY(launch_passes(ctx, p, L, np, x, y, false, s));
+        p.in = u;
+        p.out = prof + (size_t)n0 * N;
+        p.load = kLoadRows;
+        p.store = kStoreChirped;
+        SARF_TRY(launch_passes(ctx, p, L, np, x, y, false, s));
+    }
     return SARF_OK;
 }
 
@@ -790,33 +894,20 @@ int launch_range_compress(sarf_ctx *ctx, const sarf_rc_desc *d, const void *ph,
                         "power of two go up to %d)", d->Nfft, kBluesteinGlobalMaxN);
         int L = 1;
         while ((1 << L) < 2 * d->Nfft - 1) L++;
-        if (f64) {
-            const double2 *tw = nullptr;
-            SARF_TRY(twiddles_f64(ctx, L, &tw));
+        if (f64)
             return launch_bluestein_global<double2>(ctx, d, L, (const double2 *)ph, taper, f0, r0,
-                                                    tw, (double2 *)prof, s);
-        }
-        const float2 *tw = nullptr;
-        SARF_TRY(twiddles_f32(ctx, L, &tw));
-        return launch_bluestein_global<float2>(ctx, d, L, (const float2 *)ph, taper, f0, r0, tw,
+                                                    (double2 *)prof, s);
+        return launch_bluestein_global<float2>(ctx, d, L, (const float2 *)ph, taper, f0, r0,
                                                (float2 *)prof, s);
     }
     if (f64 || log2n > 14 || log2n < 5) {
         if (log2n < 1 || log2n > 24)
             return fail(SARF_ERR_UNSUPPORTED, "range_compress: Nfft=%d", d->Nfft);
-        void *tmp = nullptr;
-        if (f64) {
-            const double2 *tw = nullptr;
-            SARF_TRY(twiddles_f64(ctx, log2n, &tw));
-            SARF_TRY(scratch_get(ctx, "rc64.tmp", sizeof(double2) * (size_t)d->Nfft * d->Np, &tmp));
-            return launch_passes<double2>(d, log2n, (const double2 *)ph, taper, f0, r0, tw,
-                                          (double2 *)prof, (double2 *)tmp, s);
-        }
-        const float2 *tw = nullptr;
-        SARF_TRY(twiddles_f32(ctx, log2n, &tw));
-        SARF_TRY(scratch_get(ctx, "rc32.tmp", sizeof(float2) * (size_t)d->Nfft * d->Np, &tmp));
-        return launch_passes<float2>(d, log2n, (const float2 *)ph, taper, f0, r0, tw,
-                                     (float2 *)prof, (float2 *)tmp, s);
+        if (f64)
+            return launch_long<double2>(ctx, d, log2n, (const double2 *)ph, taper, f0, r0,
+                                        (double2 *)prof, s);
+        return launch_long<float2>(ctx, d, log2n, (const float2 *)ph, taper, f0, r0, (float2 *)prof,
+                                   s);
     }
     const float2 *tw = nullptr;
     SARF_TRY(twiddles_f32(ctx, log2n, &tw));
