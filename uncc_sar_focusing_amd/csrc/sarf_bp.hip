@@ -2,9 +2,9 @@
 //
 // bp_mixed (SARF_BP_MIXED): the tile engine of sarf_bp_core.hpp over plain
 // antenna positions, writing the image (or a per-pulse-group partial).
-// bp_f64 (SARF_BP_F64): one lane per pixel, every quantity in double, the
-// reference's search rule (cpuBackProjection.hpp:28-29) and FP64 sin/cos:
-// the "all-FP64 build" the mixed kernel is measured against at full size.
+// bp_f64 (SARF_BP_F64): every quantity in double, per pixel and pulse, with the
+// reference's interpolation rule (cpuBackProjection.hpp:28-29): the "all-FP64
+// build" the mixed kernel is measured against at full size.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -57,16 +57,18 @@ void bp_mixed(BpArgs a, const float2 *__restrict__ prof,
 }
 
 // Sums the per-split partial images in split order (deterministic) into img.
-__global__ __launch_bounds__(256) void bp_reduce_splits(const float2 *__restrict__ part,
+template <typename T2>
+__global__ __launch_bounds__(256) void bp_reduce_splits(const T2 *__restrict__ part,
                                                         long stride, int splits, long n,
-                                                        int accumulate, float2 *__restrict__ img) {
+                                                        int accumulate, T2 *__restrict__ img) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    float2 acc = accumulate ? img[i] : make_float2(0.f, 0.f);
+    T2 acc{};
+    if (accumulate) acc = img[i];
     // partials added in split order; eight loads issued before any is added
     int s = 0;
     for (; s + 8 <= splits; s += 8) {
-        float2 v[8];
+        T2 v[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) v[u] = part[(s + u) * stride + i];
 #pragma unroll
@@ -76,54 +78,124 @@ __global__ __launch_bounds__(256) void bp_reduce_splits(const float2 *__restrict
         }
     }
     for (; s < splits; s++) {
-        const float2 v = part[s * stride + i];
+        const T2 v = part[s * stride + i];
         acc.x += v.x;
         acc.y += v.y;
     }
     img[i] = acc;
 }
 
-// All-FP64 reference-precision kernel, one lane per pixel.
+// e^{j 2 pi t}, |t| <= 1/2 and a little, to about an ulp of FP64: t - q/4 in
+// [-1/8, 1/8], the Taylor polynomials of sin(2 pi x) and cos(2 pi x) there (the
+// first terms left out are below 5e-17) and a quarter turn's exchange and signs.
+__device__ __forceinline__ double2 cis_rev64(double t) {
+    const double q = rint(4.0 * t);
+    const double x = fma(-0.25, q, t), z = x * x;
+    double s = 3.8199525848482821277;
+    s = fma(z, s, -15.094642576822990392);
+    s = fma(z, s, 42.058693944897653145);
+    s = fma(z, s, -76.705859753061385842);
+    s = fma(z, s, 81.605249276075054203);
+    s = fma(z, s, -41.341702240399760234);
+    s = fma(z, s, 6.2831853071795864769);
+    s *= x;
+    double c = 0.28200596845579121507;
+    c = fma(z, c, -1.7143907110886720654);
+    c = fma(z, c, 7.9035363713184688042);
+    c = fma(z, c, -26.426256783374397453);
+    c = fma(z, c, 60.244641371876660363);
+    c = fma(z, c, -85.456817206693727736);
+    c = fma(z, c, 64.939394022668291491);
+    c = fma(z, c, -19.739208802178717238);
+    c = fma(z, c, 1.0);
+    const int k = (int)q;
+    const double a = (k & 1) ? s : c, b = (k & 1) ? c : s;
+    return make_double2(((k + 1) & 2) ? -a : a, (k & 2) ? -b : b);
+}
+
+// Square root to within an ulp of FP64: FP32 reciprocal square root, a
+// third-order step, and the remainder added back.
+__device__ __forceinline__ double sqrt_f64(double v) {
+    const double y = (double)__builtin_amdgcn_rsqf(fmaxf((float)v, 1e-30f));
+    const double g = v * y;
+    const double e = fma(-g, y, 1.0);
+    const double d = fma(g * e, fma(e, 0.375, 0.5), g);
+    return fma(fma(-d, d, v), 0.5 * y, d);
+}
+
+// All-FP64 kernel.  A workgroup (4 wave64) owns a 32 x 16 pixel tile, each wave
+// 16 x 8, a lane two pixels 8 columns apart (16 lanes in a row cover 4 x 4
+// pixels, so a wave's profile reads share cache lines); the pulses are split
+// over workgroups until the GPU is full.  Per pixel and pulse: range and
+// phase in revolutions (the product's rounding error carried along), the
+// interpolation position from the range times bins per metre, sine and cosine
+// by polynomial: about 60 instructions, two thirds of them FP64, where sqrt(),
+// sincos() and the reference's bin search with its divisions took five times
+// that.  Bound by FP64 issue: 256^2 pixels, 512 pulses 495 us (one wave per SIMD,
+// no splits) before, 100 now, the same with half the splits or two pulses
+// unrolled.
+constexpr int kF64TX = 32, kF64TY = 16;
+
 __global__ __launch_bounds__(256) void bp_f64(BpArgs a, const double2 *__restrict__ prof,
                                               const double *__restrict__ ant,
                                               const double *__restrict__ r0,
-                                              const double *__restrict__ f0,
-                                              double2 *__restrict__ img) {
-    const long pix = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (pix >= (long)a.Nx * a.Ny) return;
-    const int x = (int)(pix / a.Ny), y = (int)(pix - (long)x * a.Ny);
-    const double px = a.left + x * a.dx, py = a.bottom + y * a.dy;
+                                              const double *__restrict__ f0, double inv_bin,
+                                              double2 *__restrict__ img,
+                                              double2 *__restrict__ part) {
+    const int ntiles = a.tiles_x * a.tiles_y;
+    const int split = blockIdx.x / ntiles, t = blockIdx.x - split * ntiles;
+    const int ty = t / a.tiles_x, tx = t - ty * a.tiles_x;
+    int nbeg, nend;
+    split_range(a, split, nbeg, nend);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int x0 = tx * kF64TX + 16 * (wave & 1) + ((lane >> 2) & 3) + 4 * (lane >> 5);
+    const int y = ty * kF64TY + 8 * (wave >> 1) + (lane & 3) + 4 * ((lane >> 4) & 1);
     const int N = a.Nfft;
+    const double py = a.bottom + y * a.dy;
+    const double px[2] = {a.left + x0 * a.dx, a.left + (x0 + 8) * a.dx};
     const double rmin = -0.5 * a.maxWr, rmax = ((double)(N - 1) / N - 0.5) * a.maxWr;
-    double accr = 0.0, acci = 0.0;
-    for (int n = 0; n < a.Np; n++) {
-        const double ddx = ant[3 * n] - px, ddy = ant[3 * n + 1] - py, ddz = ant[3 * n + 2];
-        const double dR = sqrt(ddx * ddx + ddy * ddy + ddz * ddz) - r0[n];
-        if (!(dR > rmin && dR < rmax)) continue;
-        const double idx = (dR / a.maxWr + 0.5) * N;
-        int ri = (int)floor(idx) - 1;
-        if (ri < -1) ri = -1;
-        // first bin with r > dR (cpuBackProjection.hpp:28-29)
-        while (++ri < N && ((double)ri / N - 0.5) * a.maxWr <= dR) {
+    const double mid = 0.5 * N;
+    double2 acc[2] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
+    for (int n = nbeg; n < nend; n++) {
+        // wave-uniform: scalar loads
+        const double ax = ant[3 * n], ay = ant[3 * n + 1], az = ant[3 * n + 2], R0 = r0[n];
+        const double kap = f0[n] * (2.0 / kClight);  // revolutions per metre
+        const double2 *__restrict__ row = prof + (size_t)n * N;
+        const double ddy = ay - py;
+        double dR[2];
+        double2 sl[2], sr[2];
+        double al[2];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const double ddx = ax - px[j];
+            dR[j] = sqrt_f64(ddx * ddx + ddy * ddy + az * az) - R0;
+            const double pos = fma(dR[j], inv_bin, mid);
+            // r_0 < dR < r_{N-1} bounds pos to (0, N - 1) up to rounding
+            const int i = (int)fmin(fmax(pos, 0.0), (double)(N - 2));
+            al[j] = pos - (double)i;
+            sl[j] = row[i];
+            sr[j] = row[i + 1];
         }
-        if (ri == N || ri == 0) continue;
-        const double rl = ((double)(ri - 1) / N - 0.5) * a.maxWr;
-        const double rr = ((double)ri / N - 0.5) * a.maxWr;
-        const double al = (dR - rl) / (rr - rl);
-        const double2 sl = prof[(size_t)n * N + ri - 1], sr = prof[(size_t)n * N + ri];
-        const double vr = al * sr.x + (1.0 - al) * sl.x;
-        const double vi = al * sr.y + (1.0 - al) * sl.y;
-        const double ph = 4.0 * kPi * f0[n] * dR / kClight;
-        double sn, cs;
-        sincos(ph, &sn, &cs);
-        accr += vr * cs - vi * sn;
-        acci += vr * sn + vi * cs;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const double p = kap * dR[j];
+            const double2 e = cis_rev64((p - rint(p)) + fma(kap, dR[j], -p));
+            const bool ok = dR[j] > rmin && dR[j] < rmax;
+            const double vr = ok ? fma(al[j], sr[j].x - sl[j].x, sl[j].x) : 0.0;
+            const double vi = ok ? fma(al[j], sr[j].y - sl[j].y, sl[j].y) : 0.0;
+            acc[j].x = fma(vr, e.x, fma(-vi, e.y, acc[j].x));
+            acc[j].y = fma(vr, e.y, fma(vi, e.x, acc[j].y));
+        }
     }
-    double2 *o = img + pix;
-    if (a.accumulate) {
-        *o = make_double2(o->x + accr, o->y + acci);
-    } else {
-        *o = make_double2(accr, acci);
+    if (y >= a.Ny) return;
+    const bool to_part = a.splits > 1;
+    double2 *o = to_part ? part + (size_t)split * a.split_stride : img;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int x = x0 + 8 * j;
+        if (x >= a.Nx) continue;
+        const size_t idx = (size_t)x * a.Ny + y;
+        o[idx] = a.accumulate && !to_part ? cadd(o[idx], acc[j]) : acc[j];
     }
 }
 
@@ -451,7 +523,7 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
         // even groups: img (+)= sum of all partials; head + tail: the head
         // group wrote (or added into) img, the tail partials are added to it
         const int acc = a.tail > 0 || (d->flags & SARF_BP_ACCUMULATE) ? 1 : 0;
-        hipLaunchKernelGGL(bp_reduce_splits, dim3((npix + 255) / 256), dim3(256), 0, s, a.part,
+        hipLaunchKernelGGL(bp_reduce_splits<float2>, dim3((npix + 255) / 256), dim3(256), 0, s, a.part,
                            (long)npix, nparts, npix, acc, (float2 *)img);
         SARF_HIP(hipGetLastError());
     }
@@ -462,7 +534,7 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
 
 int launch_reduce_partials(const float2 *part, long stride, int splits, long n, int accumulate,
                            float2 *img, hipStream_t s) {
-    hipLaunchKernelGGL(bp_reduce_splits, dim3((n + 255) / 256), dim3(256), 0, s, part, stride,
+    hipLaunchKernelGGL(bp_reduce_splits<float2>, dim3((n + 255) / 256), dim3(256), 0, s, part, stride,
                        splits, n, accumulate, img);
     SARF_HIP(hipGetLastError());
     return SARF_OK;
@@ -480,9 +552,35 @@ int launch_backproject_ext(sarf_ctx *ctx, const sarf_bp_desc *d, const void *pro
         BpArgs a{};
         SARF_TRY(bp_fill_args(ctx, d, 0, &a));
         const long npix = (long)d->Nx * d->Ny;
-        hipLaunchKernelGGL(bp_f64, dim3((npix + 255) / 256), dim3(256), 0, s, a,
-                           (const double2 *)prof, ant, r0, f0, (double2 *)img);
+        a.tiles_x = (d->Nx + kF64TX - 1) / kF64TX;
+        a.tiles_y = (d->Ny + kF64TY - 1) / kF64TY;
+        const int ntiles = a.tiles_x * a.tiles_y;
+        // at least 8 workgroups per CU, 16 pulses or more each: the partial
+        // images of at most 4096 tiles of 512 pixels take 34 MB
+        const int want = 8 * (ctx->cu_count > 0 ? ctx->cu_count : 256);
+        while (a.splits * ntiles <= want && a.splits < 32 && d->Np / (2 * a.splits) >= 16)
+            a.splits *= 2;
+        double2 *part = nullptr;
+        if (a.splits > 1) {
+            const size_t need = sizeof(double2) * (size_t)npix * a.splits;
+            void *buf = ext_part;
+            if (!ext_part) SARF_TRY(scratch_get(ctx, "bp64.partials", need, &buf));
+            else if (need > ext_bytes)
+                return fail(SARF_ERR_INVALID, "backproject: %zu bytes of partial images, more than "
+                            "the %zu available", need, ext_bytes);
+            part = (double2 *)buf;
+            a.split_stride = npix;
+        }
+        hipLaunchKernelGGL(bp_f64, dim3((unsigned)(ntiles * a.splits)), dim3(256), 0, s, a,
+                           (const double2 *)prof, ant, r0, f0, d->Nfft / d->maxWr, (double2 *)img,
+                           part);
         SARF_HIP(hipGetLastError());
+        if (a.splits > 1) {
+            hipLaunchKernelGGL(bp_reduce_splits<double2>, dim3((unsigned)((npix + 255) / 256)),
+                               dim3(256), 0, s, part, npix, a.splits, npix, a.accumulate,
+                               (double2 *)img);
+            SARF_HIP(hipGetLastError());
+        }
         return SARF_OK;
     }
     int tile = d->tile > 0 ? d->tile : 0;
