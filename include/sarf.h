@@ -49,6 +49,8 @@ extern "C" {
 
 /* backprojection flags */
 #define SARF_BP_ACCUMULATE 1 /* add into img instead of overwriting it */
+#define SARF_BP_FOR_GRADIENT 4 /* sarf_backproject: round as sarf_bp_entropy_grad's recomputation
+                                  and sarf_bp_batch_entropy do (a little slower and coarser) */
 #define SARF_BATCH_DIR_PER_BASIS 2 /* sarf_bp_batch_entropy: dir holds one field per basis */
 #define SARF_SCENES_TILE_MIXED 100 /* sarf_bp_scenes: a tile per scene (see there) */
 
@@ -160,7 +162,7 @@ typedef struct {
     double Wx, Wy;  /* image extent (m), spacing W/(N-1) */
     double maxWr;   /* unambiguous range c/(2 mean deltaF) = max_Wy_m */
     int precision;  /* SARF_BP_MIXED | SARF_BP_F64 */
-    int flags;      /* SARF_BP_ACCUMULATE */
+    int flags;      /* SARF_BP_ACCUMULATE | SARF_BP_FOR_GRADIENT */
     int tile;       /* 0 = default for the pixel spacing and line of sight; else a
                        tile id: 1..7 (lanes along y) or 11..16 (lanes along x);
                        batches and the gradient take 1..5 and 11..16 */

@@ -131,10 +131,13 @@ class Context:
                     f0: torch.Tensor, grid: ImageGrid, maxWr: float, *,
                     precision: str = "mixed", out: torch.Tensor | None = None,
                     accumulate: bool = False, tile: int = 0,
-                    pulse_split: int = 0, los: tuple[float, float] | None = None) -> torch.Tensor:
+                    pulse_split: int = 0, los: tuple[float, float] | None = None,
+                    for_gradient: bool = False) -> torch.Tensor:
         """Backproject profiles onto `grid`.  `los` optionally gives the
         horizontal unit line of sight (x, y) from the image centre to the
-        aperture centre; it only steers the default tile shape."""
+        aperture centre; it only steers the default tile shape.
+        `for_gradient` rounds as entropy_grad's recomputation does
+        (SARF_BP_FOR_GRADIENT)."""
         Np, nfft = prof.shape
         f64 = precision == "f64"
         cdt = torch.complex128 if f64 else torch.complex64
@@ -148,7 +151,8 @@ class Context:
         _need(out, cdt, (grid.Nx, grid.Ny), "out")
         d = BpDesc(grid.Nx, grid.Ny, nfft, Np, grid.x0, grid.y0, grid.Wx, grid.Wy, maxWr,
                    _lib.SARF_BP_F64 if f64 else _lib.SARF_BP_MIXED,
-                   _lib.SARF_BP_ACCUMULATE if accumulate else 0, tile, pulse_split,
+                   (_lib.SARF_BP_ACCUMULATE if accumulate else 0)
+                   | (_lib.SARF_BP_FOR_GRADIENT if for_gradient else 0), tile, pulse_split,
                    *(los if los is not None else (0.0, 0.0)))
         check(self.lib.sarf_backproject(self._h, C.byref(d), _ptr(prof), _ptr(ant), _ptr(r0),
                                         _ptr(f0), _ptr(out), self._stream()))

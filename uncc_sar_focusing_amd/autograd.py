@@ -30,7 +30,7 @@ class BpOperator:
 
     def image(self, ant: torch.Tensor) -> torch.Tensor:
         return self.ctx.backproject(self.prof, ant.detach().contiguous(), self.r0, self.f0,
-                                    self.grid, self.maxWr, los=self.los)
+                                    self.grid, self.maxWr, los=self.los, for_gradient=True)
 
 
 class BackprojectEntropy(torch.autograd.Function):

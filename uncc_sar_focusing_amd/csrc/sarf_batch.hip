@@ -34,22 +34,23 @@ int bp_fill_args(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, BpArgs *a);
 
 namespace {
 
-template <int TY, int PX, bool XL>
-__global__ __launch_bounds__(kBpThreads) __attribute__((amdgpu_waves_per_eu(bp_waves_per_eu<TY, PX, XL>())))
+template <int TY, int PX, bool XL, int CAP>
+__global__ __launch_bounds__(kBpThreads) __attribute__((amdgpu_waves_per_eu(bp_waves_per_eu<TY, PX, XL, CAP>())))
 void bp_batch_entropy(
     BpArgs a, const float2 *__restrict__ prof, const double *__restrict__ ant,
     const double *__restrict__ r0, const double *__restrict__ f0, const double *__restrict__ dir,
     const double *__restrict__ basis, const double *__restrict__ coef, int nbasis, int ncand,
     int per_basis, double2 *__restrict__ partial) {
-    __shared__ typename BpTile<TY, PX, XL>::Lds L;
-    __shared__ __align__(16) float fx[BpTile<TY, PX, XL>::kFx];
+    using Tile = BpTile<TY, PX, XL, CAP>;
+    __shared__ typename Tile::Lds L;
+    __shared__ __align__(16) float fx[Tile::kFx];
     __shared__ double2 red[kBpThreads / 64];
     const int ntiles = a.tiles_x * a.tiles_y;
     const long nitems = (long)ntiles * ncand;
     for (long item = blockIdx.x; item < nitems; item += gridDim.x) {
         const int t = (int)(item / ncand);
         const int c = (int)(item - (long)t * ncand);
-        BpTile<TY, PX, XL> T;
+        Tile T;
         T.init(a, t);
         LosPolyPos pos{ant, dir, basis, coef + (size_t)c * nbasis, nbasis, a.Np, per_basis};
         T.run(a, L, fx, prof, pos, r0, f0, 0, a.Np);
@@ -121,12 +122,12 @@ __global__ __launch_bounds__(256) void image_entropy_final(const double2 *__rest
     }
 }
 
-template <int TY, int PX, bool XL = false>
+template <int TY, int PX, bool XL = false, int CAP = kBpCap>
 void launch_batch_t(const BpArgs &a, int grid, const float2 *prof, const double *ant,
                     const double *r0, const double *f0, const double *dir, const double *basis,
                     const double *coef, int nbasis, int ncand, int per_basis, double2 *partial,
                     hipStream_t s) {
-    hipLaunchKernelGGL((bp_batch_entropy<TY, PX, XL>), dim3(grid), dim3(kBpThreads), 0, s, a,
+    hipLaunchKernelGGL((bp_batch_entropy<TY, PX, XL, CAP>), dim3(grid), dim3(kBpThreads), 0, s, a,
                        prof, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial);
 }
 
@@ -166,9 +167,11 @@ extern "C" int sarf_bp_batch_entropy(sarf_ctx *ctx, const sarf_bp_desc *d, const
     void *buf = nullptr;
     SARF_TRY(scratch_get(ctx, "batch.partials", sizeof(double2) * (size_t)nitems, &buf));
     double2 *partial = (double2 *)buf;
-    // persistent: 4 resident workgroups per CU (LDS-limited), 2 waves of them
+    // persistent: two rounds of the resident workgroups per CU (4, or 5 where
+    // the tile's kernel has the smaller windows)
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    const int grid = (int)std::min<long>(nitems, 8L * cus);
+    const bool five = a.narrow && (tid == 13 || tid == 15 || tid == 16);
+    const int grid = (int)std::min<long>(nitems, (five ? 10L : 8L) * cus);
     hipStream_t s = (hipStream_t)stream;
     const float2 *p = (const float2 *)prof;
     switch (tid) {
@@ -179,10 +182,19 @@ extern "C" int sarf_bp_batch_entropy(sarf_ctx *ctx, const sarf_bp_desc *d, const
         case 5: launch_batch_t<16, 4>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
         case 11: launch_batch_t<32, 4, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
         case 12: launch_batch_t<64, 4, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
-        case 13: launch_batch_t<64, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
+        case 13:
+            if (a.narrow) launch_batch_t<64, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            else launch_batch_t<64, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            break;
         case 14: launch_batch_t<32, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
-        case 15: launch_batch_t<256, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
-        case 16: launch_batch_t<128, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
+        case 15:
+            if (a.narrow) launch_batch_t<256, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            else launch_batch_t<256, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            break;
+        case 16:
+            if (a.narrow) launch_batch_t<128, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            else launch_batch_t<128, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            break;
         default:
             return fail(SARF_ERR_UNSUPPORTED, "sarf_bp_batch_entropy: tile %d not compiled for batches", tid);
     }

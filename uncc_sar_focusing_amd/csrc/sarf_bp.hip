@@ -15,34 +15,27 @@
 namespace sarf {
 namespace {
 
-template <int TY, int PX, bool XL>
-__global__ __launch_bounds__(kBpThreads) __attribute__((amdgpu_waves_per_eu(bp_waves_per_eu<TY, PX, XL>())))
-void bp_mixed(BpArgs a, const float2 *__restrict__ prof,
-                                                       const double *__restrict__ ant,
-                                                       const double *__restrict__ r0,
-                                                       const double *__restrict__ f0,
-                                                       float2 *__restrict__ img) {
-    __shared__ typename BpTile<TY, PX, XL>::Lds L;
-    __shared__ __align__(16) float fx[BpTile<TY, PX, XL>::kFx];
-    // blockIdx.x = split * ntiles + tile: every split of a tile covers a
-    // contiguous pulse range and writes its own partial image -- except the
-    // head group of a head + tail split, which writes the image itself
+// blockIdx.x = split * ntiles + tile: every split of a tile covers a contiguous
+// pulse range and writes its own partial image -- except the head group of a
+// head + tail split, which writes the image itself.
+__device__ __forceinline__ int split_block(const BpArgs &a, float2 *&img, int &accumulate, int &nbeg,
+                                           int &nend) {
     const int ntiles = a.tiles_x * a.tiles_y;
     const int split = blockIdx.x / ntiles;
-    const int t = swizzle_tile(blockIdx.x - split * ntiles, ntiles);
-    int nbeg, nend;
     split_range(a, split, nbeg, nend);
-    int accumulate = a.accumulate;
+    accumulate = a.accumulate;
     if (a.splits > 1 && !(a.tail > 0 && split == 0)) {
         img = a.part + (size_t)(a.tail > 0 ? split - 1 : split) * a.split_stride;
         accumulate = 0;
     }
+    return swizzle_tile(blockIdx.x - split * ntiles, ntiles);
+}
 
-    BpTile<TY, PX, XL> T;
-    T.init(a, t);
-    T.run(a, L, fx, prof, PlainPos{ant}, r0, f0, nbeg, nend);
+template <class Tile>
+__device__ __forceinline__ void store_tile(const Tile &T, const BpArgs &a, float2 *img,
+                                           int accumulate) {
 #pragma unroll
-    for (int j = 0; j < PX; j++) {
+    for (int j = 0; j < Tile::kPx; j++) {
         int x, y;
         if (T.pixel(j, x, y, a)) {
             float2 *o = img + (size_t)x * a.Ny + y;
@@ -54,6 +47,41 @@ void bp_mixed(BpArgs a, const float2 *__restrict__ prof,
             }
         }
     }
+}
+
+template <int TY, int PX, bool XL, int CAP>
+__global__ __launch_bounds__(kBpThreads) __attribute__((amdgpu_waves_per_eu(bp_waves_per_eu<TY, PX, XL, CAP>())))
+void bp_mixed(BpArgs a, const float2 *__restrict__ prof,
+                                                       const double *__restrict__ ant,
+                                                       const double *__restrict__ r0,
+                                                       const double *__restrict__ f0,
+                                                       float2 *__restrict__ img) {
+    using Tile = BpTile<TY, PX, XL, CAP>;
+    __shared__ typename Tile::Lds L;
+    __shared__ __align__(16) float fx[Tile::kFx];
+    int nbeg, nend, accumulate;
+    float2 *out = img;
+    const int t = split_block(a, out, accumulate, nbeg, nend);
+    Tile T;
+    T.init(a, t);
+    T.run(a, L, fx, prof, PlainPos{ant}, r0, f0, nbeg, nend);
+    store_tile(T, a, out, accumulate);
+}
+
+// The same over BpTileU.
+template <int TL, int PX, bool XL>
+__global__ __launch_bounds__(kBpThreads) __attribute__((amdgpu_waves_per_eu(kBpWavesU)))
+void bp_mixed_u(BpArgs a, const float2 *__restrict__ prof, const double *__restrict__ ant,
+                const double *__restrict__ r0, const double *__restrict__ f0,
+                float2 *__restrict__ img) {
+    __shared__ typename BpTileU<TL, PX, XL>::Lds L;
+    int nbeg, nend, accumulate;
+    float2 *out = img;
+    const int t = split_block(a, out, accumulate, nbeg, nend);
+    BpTileU<TL, PX, XL> T;
+    T.init(a, t);
+    T.run(a, L, nullptr, prof, PlainPos{ant}, r0, f0, nbeg, nend);
+    store_tile(T, a, out, accumulate);
 }
 
 // Sums the per-split partial images in split order (deterministic) into img.
@@ -226,10 +254,17 @@ constexpr TileShape kTiles[] = {
     {16, 128, 16, 128, 8, 1},
 };
 
-template <int TY, int PX, bool XL = false>
+template <int TY, int PX, bool XL = false, int CAP = kBpCap>
 void launch_mixed_t(const BpArgs &a, int grid, const float2 *prof, const double *ant,
                     const double *r0, const double *f0, float2 *img, hipStream_t s) {
-    hipLaunchKernelGGL((bp_mixed<TY, PX, XL>), dim3(grid), dim3(kBpThreads), 0, s, a, prof, ant,
+    hipLaunchKernelGGL((bp_mixed<TY, PX, XL, CAP>), dim3(grid), dim3(kBpThreads), 0, s, a, prof, ant,
+                       r0, f0, img);
+}
+
+template <int TL, int PX, bool XL>
+void launch_mixed_u(const BpArgs &a, int grid, const float2 *prof, const double *ant,
+                    const double *r0, const double *f0, float2 *img, hipStream_t s) {
+    hipLaunchKernelGGL((bp_mixed_u<TL, PX, XL>), dim3(grid), dim3(kBpThreads), 0, s, a, prof, ant,
                        r0, f0, img);
 }
 
@@ -375,7 +410,8 @@ int bp_fill_args(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, BpArgs *out) {
     a.left = d->x0 - d->Wx / 2;
     a.bottom = d->y0 - d->Wy / 2;
     a.maxWr = d->maxWr;
-    a.invbin = (float)(d->Nfft / d->maxWr);
+    a.binv = d->Nfft / d->maxWr;
+    a.invbin = (float)a.binv;
     a.splits = 1;
     a.tail = 0;
     a.split_stride = 0;
@@ -390,6 +426,7 @@ int bp_fill_args(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, BpArgs *out) {
             return fail(SARF_ERR_UNSUPPORTED,
                         "backproject: tile %d spans %.0f range bins (> %d); pixel spacing too "
                         "coarse for the range bin width", tile, wmax, kBpCap);
+        a.narrow = wmax <= kBpCapX;
         a.tiles_x = (d->Nx + tx - 1) / tx;
         a.tiles_y = (d->Ny + ty - 1) / ty;
     }
@@ -502,6 +539,10 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
     }
     const int grid = ntiles * splits;
     const float2 *p = (const float2 *)prof;
+    // Tile 15: BpTileU, except for the image a gradient is taken of, whose
+    // rounding the adjoint kernel repeats, and where BpTile's larger windows
+    // are needed
+    const bool for_gradient = (d->flags & SARF_BP_FOR_GRADIENT) != 0;
     switch (tid) {
         case 1: launch_mixed_t<32, 4>(a, grid, p, ant, r0, f0, o, s); break;
         case 2: launch_mixed_t<64, 4>(a, grid, p, ant, r0, f0, o, s); break;
@@ -512,10 +553,20 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
         case 7: launch_mixed_t<32, 16>(a, grid, p, ant, r0, f0, o, s); break;
         case 11: launch_mixed_t<32, 4, true>(a, grid, p, ant, r0, f0, o, s); break;
         case 12: launch_mixed_t<64, 4, true>(a, grid, p, ant, r0, f0, o, s); break;
-        case 13: launch_mixed_t<64, 8, true>(a, grid, p, ant, r0, f0, o, s); break;
+        case 13:
+            if (a.narrow) launch_mixed_t<64, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
+            else launch_mixed_t<64, 8, true>(a, grid, p, ant, r0, f0, o, s);
+            break;
         case 14: launch_mixed_t<32, 8, true>(a, grid, p, ant, r0, f0, o, s); break;
-        case 15: launch_mixed_t<256, 8, true>(a, grid, p, ant, r0, f0, o, s); break;
-        case 16: launch_mixed_t<128, 8, true>(a, grid, p, ant, r0, f0, o, s); break;
+        case 15:
+            if (!a.narrow) launch_mixed_t<256, 8, true>(a, grid, p, ant, r0, f0, o, s);
+            else if (for_gradient) launch_mixed_t<256, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
+            else launch_mixed_u<256, 8, true>(a, grid, p, ant, r0, f0, o, s);
+            break;
+        case 16:
+            if (a.narrow) launch_mixed_t<128, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
+            else launch_mixed_t<128, 8, true>(a, grid, p, ant, r0, f0, o, s);
+            break;
         default: return fail(SARF_ERR_INVALID, "backproject: unknown tile id %d", tid);
     }
     SARF_HIP(hipGetLastError());

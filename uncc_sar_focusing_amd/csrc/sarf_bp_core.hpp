@@ -55,22 +55,27 @@
 namespace sarf {
 
 constexpr int kBpThreads = 256;
+constexpr int kBpChunk = 32;  // max pulses staged per chunk (the 256-lane tile stages 64)
+constexpr int kBpCap = 2048;  // LDS window capacity, in bins (16 B each)
+// The same of kernels for geometries whose windows are never wider, so that
+// five workgroups fit in a CU's LDS.
+constexpr int kBpCapX = 1536;
+static_assert(kBpChunk <= 64 && kBpCap % kBpThreads == 0, "staging layout");
+
 // Waves per SIMD the tile kernels are compiled for: 4 (<= 128 VGPRs) up to
 // 8 pixels per lane, except lanes-along-x tiles whose column terms take the
 // LDS past 40 KiB (3 workgroups per CU); the 16-pixel tiles need more
-// registers than that.
-template <int TY, int PX, bool XL>
+// registers than that.  Tiles 13, 15 and 16 with the smaller windows: 5 (2048^2
+// at 0.05 m, 4096 pulses, tile 16 6.98 -> 6.74 ms, tile 13 7.23 -> 6.94; 1331
+// candidates at 512^2, 1024 pulses, tile 15 154.0 -> 150.2 ms, 153.7 with 4).
+template <int TY, int PX, bool XL, int CAP = kBpCap>
 constexpr int bp_waves_per_eu() {
-    return PX > 8 ? 1 : (XL && (kBpThreads / TY) * PX > 32) ? 3 : 4;
+    return CAP < kBpCap ? 5 : PX > 8 ? 1 : (XL && (kBpThreads / TY) * PX > 32) ? 3 : 4;
 }
 // The same for a tile described at run time (lanes tl, pixels per lane px).
 constexpr int bp_waves_per_eu_rt(int tl, int px, bool xl) {
     return px > 8 ? 1 : (xl && (kBpThreads / tl) * px > 32) ? 3 : 4;
 }
-constexpr int kBpChunk = 32;  // max pulses staged per chunk (the 256-lane tile stages 64)
-constexpr int kBpCap = 2048;  // LDS window capacity, in bins (16 B each)
-static_assert(kBpChunk <= 64 && kBpCap % kBpThreads == 0, "staging layout");
-
 struct BpArgs {
     int Nx, Ny, Nfft, Np;
     int tiles_x, tiles_y;
@@ -84,6 +89,8 @@ struct BpArgs {
     double left, bottom, dx, dy;  // pixel (i,j) = (left + i dx, bottom + j dy)
     double maxWr;
     float invbin;  // Nfft / maxWr (bins per metre)
+    double binv;   // the same in FP64
+    int narrow;    // no window of the tile is wider than kBpCapX
 };
 
 // Pulse range [nbeg, nend) of split s of a tile: even groups, or, with a
@@ -108,11 +115,11 @@ __device__ __forceinline__ void split_range(const BpArgs &a, int s, int &nbeg, i
     nend = min(a.Np, nbeg + per);
 }
 
-// Staged state of one chunk of up to CH pulses.
-template <int CH>
+// Staged state of one chunk of up to CH pulses, CAP window bins.
+template <int CH, int CAP>
 struct BpLdsT {
     static_assert(CH <= 64, "one wave stages a chunk");
-    float4 win[kBpCap];
+    float4 win[CAP];
     float4 pA[CH];  // uh_x, uh_y, g0, g1
     float4 pB[CH];  // pos_c (window-local), psi_c, kappa, W - 2
     int4 pI[CH];    // start bin, LDS offset (bins), W, interior
@@ -168,10 +175,54 @@ __device__ __forceinline__ int swizzle_tile(int b, int ntiles) {
     return (b & 7) * per + (b >> 3);
 }
 
+// Bins of a tile's windows, staged by the whole workgroup: bin f of the
+// packed windows belongs to the last pulse c with offset <= f (pI.y), profile
+// bin pI.x + f - pI.y; the chunk's first profile is `base`.  In rounds of
+// kSlots bins per thread whose loads are all issued before any is consumed.
+template <int CH>
+__device__ __forceinline__ void fill_windows(float4 *win, const int4 *pI, int nc, int tot,
+                                             const float2 *__restrict__ base, int Nfft) {
+    const int tid = threadIdx.x;
+    constexpr int kSlots = 4;
+    for (int f0r = 0; f0r < tot; f0r += kSlots * kBpThreads) {
+        float2 v0[kSlots], v1[kSlots];
+        int wb[kSlots];
+#pragma unroll
+        for (int k = 0; k < kSlots; k++) {
+            const int f = f0r + tid + k * kBpThreads;
+            v0[k] = make_float2(0.f, 0.f);
+            v1[k] = make_float2(0.f, 0.f);
+            wb[k] = 0;
+            if (f < tot) {
+                int c = 0;
+#pragma unroll
+                for (int step = CH / 2; step >= 1; step >>= 1)
+                    if (c + step < nc && pI[c + step].y <= f) c += step;
+                const int4 I = pI[c];
+                const int b = f - I.y;
+                const int g = I.x + b;  // profile bin; |g| < 2 Nfft
+                const unsigned o = (unsigned)(c * Nfft + g);  // < CH * Nfft
+                if (g >= 0 && g < Nfft) v0[k] = base[o];
+                if (g + 1 >= 0 && g + 1 < Nfft) v1[k] = base[o + 1];
+                wb[k] = b;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kSlots; k++) {
+            const int f = f0r + tid + k * kBpThreads;
+            if (f < tot) {
+                const float dr = v1[k].x - v0[k].x, di = v1[k].y - v0[k].y;
+                const float fb = (float)wb[k];
+                win[f] = make_float4(fmaf(-fb, dr, v0[k].x), fmaf(-fb, di, v0[k].y), dr, di);
+            }
+        }
+    }
+}
+
 // XL = false: the TY lanes of a group run along y and each lane owns PX
 // pixels along x (tile (256/TY * PX) x TY).  XL = true: the TY lanes run
 // along x and each lane owns PX pixels along y (tile TY x (256/TY * PX)).
-template <int TY, int PX, bool XL = false>
+template <int TY, int PX, bool XL = false, int CAP = kBpCap>
 struct BpTile {
     static constexpr int TL = TY;                  // lanes along the lane axis
     static constexpr int GX = kBpThreads / TL;     // lane groups along the pixel axis
@@ -184,12 +235,18 @@ struct BpTile {
     // 8-column F_p table leave room for them within four workgroups' LDS per
     // CU (fewer chunk rounds: 2048^2 x 4096 pulses 6.88 -> 6.71 ms), 32 else.
     static constexpr int CH = (XL && TL == 256 && PX <= 8) ? 64 : kBpChunk;
-    using Lds = BpLdsT<CH>;
+    using Lds = BpLdsT<CH, CAP>;
     static constexpr int kFx = kSep ? CH * NP : 4;  // LDS floats for F_p
     int ix0, iy0, ly, gx;
     double pcx, pcy, hx, hy;
     float qy;  // lane coordinate, tile-centred (y if !XL, x if XL)
     float qx[PX], q2[PX], x2[PX], accr[PX], acci[PX];  // pixel-axis coordinates
+
+    // With 64 lanes or more along the lane axis a wave has one range of
+    // pixel-axis coordinates: scalar registers instead of 2 PX vector registers.
+    static __device__ __forceinline__ float uniform(float v) {
+        return TL >= 64 ? __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))) : v;
+    }
 
     __device__ __forceinline__ void init(const BpArgs &a, int t) {
         const int ty = t / a.tiles_x, tx = t - ty * a.tiles_x;
@@ -201,14 +258,14 @@ struct BpTile {
         hy = 0.5 * (TYE - 1) * a.dy;
         const int tid = threadIdx.x;
         ly = tid % TL;
-        gx = tid / TL;
+        gx = TL >= 64 ? __builtin_amdgcn_readfirstlane(tid / TL) : tid / TL;
         const double dl = XL ? a.dx : a.dy, dp = XL ? a.dy : a.dx;
         qy = (float)((ly - 0.5 * (TL - 1)) * dl);
 #pragma unroll
         for (int j = 0; j < PX; j++) {
-            qx[j] = (float)((gx * PX + j - 0.5 * (NP - 1)) * dp);
+            qx[j] = uniform((float)((gx * PX + j - 0.5 * (NP - 1)) * dp));
             q2[j] = qx[j] * qx[j] + qy * qy;
-            x2[j] = qx[j] * qx[j];
+            x2[j] = uniform(qx[j] * qx[j]);
             accr[j] = 0.f;
             acci[j] = 0.f;
         }
@@ -251,7 +308,7 @@ struct BpTile {
             const long st = (long)floor(posg - span) - 1;
             // Clamped so a pulse always fits; the host checks the worst case so
             // the clamp does not bind for valid geometry.
-            W = min((int)((long)ceil(posg + span) - st) + 2, kBpCap);
+            W = min((int)((long)ceil(posg + span) - st) + 2, CAP);
             start = (int)st;
             const double kap = 2.0 * f0[n] / kClight;  // revolutions per metre
             double psi = kap * dRc;
@@ -291,7 +348,7 @@ struct BpTile {
                 const int t = __shfl_up(incl, d, 64);
                 if (tid >= d) incl += t;
             }
-            const int nc = __popcll(__ballot(tid < cmax && incl <= kBpCap));
+            const int nc = __popcll(__ballot(tid < cmax && incl <= CAP));
             if (tid < cmax) L.pI[tid] = make_int4(start, incl - W, W, interior);
             if (tid == nc - 1) {
                 L.nc = nc;
@@ -300,45 +357,7 @@ struct BpTile {
         }
         __syncthreads();
         const int nc = L.nc, tot = L.tot;
-        // Window fill over the chunk's bins as one flat range, in rounds of
-        // kSlots bins per thread whose loads are all issued before any is
-        // consumed (one memory latency per round instead of one per pulse):
-        // bin f belongs to the last pulse c with offset <= f.
-        constexpr int kSlots = 4;
-        const float2 *__restrict__ base = prof + (size_t)n0 * a.Nfft;  // chunk's first profile
-        for (int f0r = 0; f0r < tot; f0r += kSlots * kBpThreads) {
-            float2 v0[kSlots], v1[kSlots];
-            int wb[kSlots];
-#pragma unroll
-            for (int k = 0; k < kSlots; k++) {
-                const int f = f0r + tid + k * kBpThreads;
-                v0[k] = make_float2(0.f, 0.f);
-                v1[k] = make_float2(0.f, 0.f);
-                wb[k] = 0;
-                if (f < tot) {
-                    int c = 0;
-#pragma unroll
-                    for (int step = CH / 2; step >= 1; step >>= 1)
-                        if (c + step < nc && L.pI[c + step].y <= f) c += step;
-                    const int4 I = L.pI[c];
-                    const int b = f - I.y;
-                    const int g = I.x + b;  // profile bin; |g| < 2 Nfft
-                    const unsigned o = (unsigned)(c * a.Nfft + g);  // < CH * Nfft
-                    if (g >= 0 && g < a.Nfft) v0[k] = base[o];
-                    if (g + 1 >= 0 && g + 1 < a.Nfft) v1[k] = base[o + 1];
-                    wb[k] = b;
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < kSlots; k++) {
-                const int f = f0r + tid + k * kBpThreads;
-                if (f < tot) {
-                    const float dr = v1[k].x - v0[k].x, di = v1[k].y - v0[k].y;
-                    const float fb = (float)wb[k];
-                    L.win[f] = make_float4(fmaf(-fb, dr, v0[k].x), fmaf(-fb, di, v0[k].y), dr, di);
-                }
-            }
-        }
+        fill_windows<CH>(L.win, L.pI, nc, tot, prof + (size_t)n0 * a.Nfft, a.Nfft);
         if (kSep && fx != nullptr) {
             static_assert(kBpThreads % NP == 0, "a thread keeps one column");
             const int col = tid % NP;
@@ -384,18 +403,24 @@ struct BpTile {
             }
             const float wmax = B.w;
             if (I.w) {
-                // interior: no gate, no clamp (as in accumulate_chunk)
+                // interior: no gate, no clamp (as in accumulate_chunk); every
+                // window read of the pulse is issued before the first is used
+                float p[PX], ph[PX];
+                float4 w[PX];
 #pragma unroll
                 for (int j = 0; j < PX; j++) {
                     const float dl = fmaf(x2[j], C2, fmaf(qx[j], C1, F[j]));
-                    const float p = fmaf(dl, invbin, bx);
-                    const int i = (int)p;
-                    const float4 w = L.win[I.y + i];
-                    const float vr = fmaf(p, w.z, w.x);
-                    const float vi = fmaf(p, w.w, w.y);
-                    const float ph = fmaf(dl, B.z, by);  // revolutions
-                    const float sn = __builtin_amdgcn_sinf(ph);
-                    const float cs = __builtin_amdgcn_cosf(ph);
+                    p[j] = fmaf(dl, invbin, bx);
+                    ph[j] = fmaf(dl, B.z, by);  // revolutions
+                    w[j] = L.win[I.y + (int)p[j]];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < PX; j++) {
+                    const float vr = fmaf(p[j], w[j].z, w[j].x);
+                    const float vi = fmaf(p[j], w[j].w, w[j].y);
+                    const float sn = __builtin_amdgcn_sinf(ph[j]);
+                    const float cs = __builtin_amdgcn_cosf(ph[j]);
                     accr[j] = fmaf(vr, cs, fmaf(-vi, sn, accr[j]));
                     acci[j] = fmaf(vr, sn, fmaf(vi, cs, acci[j]));
                 }
@@ -499,6 +524,275 @@ struct BpTile {
             stage(a, L, prof, pos, r0, f0, n0, min(CH, nend - n0), fx);
             accumulate_chunk(a, L, fx);
             n0 += L.nc;
+        }
+    }
+};
+
+// ---------------------------------------------------------------------------
+// BpTileU: tiles whose waves have one range of pixel-axis coordinates each (64
+// lanes or more along the lane axis), for image formation.  Same expansion of
+// the range as BpTile, kept in revolutions and regrouped around the middle of
+// the wave's PX pixels (P = Pc + d in pixel spacings, d = +-1/2, +-3/2, .., so
+// instruction literals):
+//   phase(d) = by + d^2 kB + d kA,
+//   by = psi_c + rev(L, Pc), kA, kB its slope and half its curvature along P,
+// per (pulse, lane) 11 instructions; then a pair of pixels +-d shares
+// by + d^2 kB, and the window position follows from the phase,
+//   p = phase * bins_per_revolution + bx,
+// so a pixel takes 2.5 FMA for phase and position where the separable form of
+// BpTile takes 4 and two LDS reads.  by is reduced to one revolution first,
+// which leaves the phase a few revolutions at most: its rounding (the
+// error of the image) is no larger than before.
+// Pulses whose window or phase needs it take the gated form of the same.  The
+// direct expansion over the profile in memory remains for pulses whose window
+// does not fit in LDS, that are so near that the cubic term along the pixel
+// axis (left out here) would show, or that have no carrier to speak of.
+// Bound by VALU issue: 97 instructions and 16 sines and cosines per 8 pixels and
+// pulse where BpTile takes 109 and 16.  It hides its LDS latencies only with
+// five waves per SIMD (kBpCapX is what five workgroups' LDS leaves; 96 VGPRs):
+// 2048^2 at 0.05 m, 4096 pulses, tile 15: BpTile 6.75 ms, this with four waves
+// 6.25, with five 5.85 (2.9 T pixel-pulses/s; six waves the same), and rel-L2
+// against FP64 2.7e-6 -> 1.8e-6.  With 16 pixels per lane (107 instructions per
+// 8 pixels, 128 VGPRs, four waves) 6.29.  Only tile 15: tiles 16 and 13 keep
+// the rounding of BpTile, which is most of what their images are off by.
+// ---------------------------------------------------------------------------
+enum : int { kPulseFast = 0, kPulseGated = 1, kPulseDirect = 2 };
+constexpr int kBpWavesU = 5;  // waves per SIMD (workgroups per CU)
+
+template <int CH>
+struct BpLdsU {
+    static_assert(CH <= 64, "one wave stages a chunk");
+    float4 win[kBpCapX];
+    // (k: revolutions per metre; w: pixel spacing along the pixel axis)
+    float4 qA[CH];  // -k u_l, k c2l, k c3l, psi_c
+    float4 qB[CH];  // -k w u_p, k w e1, k w e2, k w^2 c2p
+    float4 qC[CH];  // k w^2 e3, bins per revolution, pos_c, LDS offset (bins, as int)
+    int4 pI[CH];    // start bin, LDS offset, W, kPulse*
+    float4 pA[CH];  // direct form: uh_x, uh_y, g0, g1
+    float kap[CH];
+    int nc, tot, fast;  // pulses staged, window bins staged, all of them kPulseFast
+};
+
+template <int TL_, int PX, bool XL>
+struct BpTileU {
+    static constexpr int TL = TL_;
+    static constexpr int GX = kBpThreads / TL;
+    static constexpr int NP = GX * PX;
+    static constexpr int kPx = PX;
+    static constexpr int TX = XL ? TL : NP;
+    static constexpr int TYE = XL ? NP : TL;
+    static constexpr int CH = TL == 256 ? 64 : kBpChunk;
+    static_assert(TL % 64 == 0 && PX % 2 == 0, "one range of pixel coordinates per wave");
+    using Lds = BpLdsU<CH>;
+    static constexpr int kFx = 4;  // no per-column terms (BpTile's interface)
+    int ix0, iy0, ly, gx;
+    double pcx, pcy, hx, hy;
+    float ql;  // lane coordinate, tile-centred
+    float Pc;  // middle of the wave's pixels in pixel spacings (uniform)
+    float accr[PX], acci[PX];
+
+    __device__ __forceinline__ void init(const BpArgs &a, int t) {
+        const int ty = t / a.tiles_x, tx = t - ty * a.tiles_x;
+        ix0 = tx * TX;
+        iy0 = ty * TYE;
+        pcx = a.left + (ix0 + 0.5 * (TX - 1)) * a.dx;
+        pcy = a.bottom + (iy0 + 0.5 * (TYE - 1)) * a.dy;
+        hx = 0.5 * (TX - 1) * a.dx;
+        hy = 0.5 * (TYE - 1) * a.dy;
+        ly = threadIdx.x % TL;
+        gx = __builtin_amdgcn_readfirstlane(threadIdx.x / TL);
+        ql = (float)((ly - 0.5 * (TL - 1)) * (XL ? a.dx : a.dy));
+        Pc = (float)(gx * PX) + 0.5f * (PX - NP);
+#pragma unroll
+        for (int j = 0; j < PX; j++) accr[j] = acci[j] = 0.f;
+    }
+
+    __device__ __forceinline__ bool pixel(int j, int &x, int &y, const BpArgs &a) const {
+        x = XL ? ix0 + ly : ix0 + gx * PX + j;
+        y = XL ? iy0 + gx * PX + j : iy0 + ly;
+        return x < a.Nx && y < a.Ny;
+    }
+
+    template <class Pos>
+    __device__ __forceinline__ void stage(const BpArgs &a, Lds &L, const float2 *__restrict__ prof,
+                                          const Pos &pos, const double *__restrict__ r0,
+                                          const double *__restrict__ f0, int n0, int cmax) {
+        const int tid = threadIdx.x;
+        __syncthreads();  // previous users of L are done
+        if (tid < 64) {
+            // one lane per pulse of the chunk (cmax <= CH <= 64); the set-up,
+            // window bound and packing of BpTile::stage
+            int W = 0, start = 0, mode = kPulseFast;
+            float4 C = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (tid < cmax) {
+                const int n = n0 + tid;
+                const double3 an = pos(n);
+                const double ux = an.x - pcx, uy = an.y - pcy, uz = an.z;
+                const double Rc = sqrt(ux * ux + uy * uy + uz * uz);
+                const double iR = 1.0 / Rc;
+                const double dRc = Rc - r0[n];
+                const double posg = fma(dRc, a.binv, 0.5 * a.Nfft);
+                const double ext = fabs(ux * iR) * hx + fabs(uy * iR) * hy + (hx * hx + hy * hy) * 0.5 * iR;
+                const double span = ext * a.binv;
+                const double st = floor(posg - span) - 1.0;
+                const double wd = ceil(posg + span) - st + 2.0;
+                start = (int)st;
+                const double kap = f0[n] * (2.0 / kClight);
+                double psi = kap * dRc;
+                psi -= rint(psi);
+                const double ah = ux * iR, bh = uy * iR, g0 = 0.5 * iR, g1 = 0.5 * iR * iR;
+                const double up = XL ? bh : ah, ul = XL ? ah : bh;
+                const double mp = 1.0 - up * up, ml = 1.0 - ul * ul;
+                L.qA[tid] = make_float4((float)(-kap * ul), (float)(kap * g0 * ml),
+                                        (float)(kap * g1 * ul * ml), (float)psi);
+                const double w = XL ? a.dy : a.dx, kw = kap * w;
+                L.qB[tid] = make_float4((float)(-kw * up), (float)(-2.0 * kw * up * ul * g0),
+                                        (float)(kw * g1 * up * (1.0 - 3.0 * ul * ul)),
+                                        (float)(kw * w * g0 * mp));
+                C = make_float4((float)(kw * w * g1 * ul * (1.0 - 3.0 * up * up)),
+                                (float)(a.binv / kap), (float)(posg - st), 0.f);
+                L.pA[tid] = make_float4((float)ah, (float)bh, (float)g0, (float)g1);
+                L.kap[tid] = (float)kap;
+                const bool inside = st >= 0.0 && st + wd <= a.Nfft && kap * ext <= 250.0;
+                mode = inside ? kPulseFast : kPulseGated;
+                // half extent along the pixel axis; the cubic term there in
+                // revolutions, and a carrier so low that the phase cannot
+                // carry the position
+                const double hp = XL ? hy : hx;
+                if (!(wd <= kBpCapX) || !(fabs(kap) * g1 * hp * hp * hp <= 1e-6) ||
+                    !(fabsf(C.y) <= 1e4f))
+                    mode = kPulseDirect;
+                else
+                    W = (int)wd;
+            }
+            int incl = W;
+#pragma unroll
+            for (int d = 1; d < CH; d <<= 1) {
+                const int t = __shfl_up(incl, d, 64);
+                if (tid >= d) incl += t;
+            }
+            const int nc = __popcll(__ballot(tid < cmax && incl <= kBpCapX));
+            const bool slow = __ballot(tid < nc && mode != kPulseFast) != 0;
+            if (tid < cmax) {
+                C.w = __int_as_float(incl - W);
+                L.qC[tid] = C;
+                L.pI[tid] = make_int4(start, incl - W, W, mode);
+            }
+            if (tid == nc - 1) {
+                L.nc = nc;
+                L.tot = incl;
+                L.fast = slow ? 0 : 1;
+            }
+        }
+        __syncthreads();
+        fill_windows<CH>(L.win, L.pI, L.nc, L.tot, prof + (size_t)n0 * a.Nfft, a.Nfft);
+        __syncthreads();
+    }
+
+    // One staged pulse, kPulseFast or kPulseGated.
+    template <bool GATED>
+    __device__ __forceinline__ void pulse(const BpArgs &a, const Lds &L, int c) {
+        const float4 A = L.qA[c];
+        const float4 B = L.qB[c];
+        const float4 C = L.qC[c];
+        const float kB = fmaf(ql, C.x, B.w);
+        float kA = fmaf(ql, fmaf(ql, B.z, B.y), B.x);
+        float rev = ql * fmaf(ql, fmaf(ql, A.z, A.y), A.x);
+        if constexpr (GX > 1) {
+            rev = fmaf(Pc, fmaf(Pc, kB, kA), rev);
+            kA = fmaf(2.f * Pc, kB, kA);
+        }
+        const float by = __builtin_amdgcn_fractf(A.w + rev);
+        // window position at phase 0 of the reduced phase
+        const float bx = fmaf(C.y, rev - by, C.z);
+        const float4 *win = L.win + __float_as_int(C.w);
+        float glo = 0.f, ghi = 0.f, wmax = 0.f;
+        if constexpr (GATED) {
+            const int4 I = L.pI[c];
+            glo = (float)(-I.x);
+            ghi = (float)(a.Nfft - 1 - I.x);
+            wmax = (float)(I.z - 2);
+        }
+        // every window read of the pulse is issued before the first is used (left
+        // alone the compiler waits for each in turn: 5.94 against 5.87 ms)
+        float ph[PX], p[PX];
+        float4 w[PX];
+#pragma unroll
+        for (int j = 0; j < PX; j++) {
+            const float d = j - 0.5f * (PX - 1);
+            ph[j] = fmaf(d, kA, fmaf(d * d, kB, by));
+            p[j] = fmaf(ph[j], C.y, bx);
+            // fast: the window has a bin of margin on each side, 1 <= p <= W - 2
+            w[j] = win[GATED ? (int)__builtin_amdgcn_fmed3f(p[j], 0.f, wmax) : (int)p[j]];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < PX; j++) {
+            const bool ok = !GATED || (p[j] > glo && p[j] < ghi);
+            const float vr = ok ? fmaf(p[j], w[j].z, w[j].x) : 0.f;
+            const float vi = ok ? fmaf(p[j], w[j].w, w[j].y) : 0.f;
+            const float rev = GATED ? __builtin_amdgcn_fractf(ph[j]) : ph[j];
+            const float sn = __builtin_amdgcn_sinf(rev);
+            const float cs = __builtin_amdgcn_cosf(rev);
+            accr[j] = fmaf(vr, cs, fmaf(-vi, sn, accr[j]));
+            acci[j] = fmaf(vr, sn, fmaf(vi, cs, acci[j]));
+        }
+    }
+
+    // One pulse by the direct expansion from its profile in memory, gated.
+    __device__ __forceinline__ void pulse_direct(const BpArgs &a, const Lds &L, int c,
+                                                 const float2 *__restrict__ row) {
+        const float4 A = L.pA[c];
+        const int start = L.pI[c].x;
+        const float kap = L.kap[c], psi = L.qA[c].w, pos = L.qC[c].z;
+        const float ul = XL ? A.x : A.y, up = XL ? A.y : A.x;
+        const float glo = (float)(-start), ghi = (float)(a.Nfft - 1 - start);
+        // opaque, so that this path's per-pixel constants are not held in
+        // registers through the others
+        float dp = (float)(XL ? a.dy : a.dx), mid = Pc;
+        __asm__ volatile("" : "+v"(dp), "+v"(mid));
+#pragma unroll
+        for (int j = 0; j < PX; j++) {
+            const float P = (mid + (j - 0.5f * (PX - 1))) * dp;
+            const float s = fmaf(up, P, ul * ql);
+            const float t = fmaf(-s, s, fmaf(P, P, ql * ql));
+            const float dl = fmaf(t, fmaf(s, A.w, A.z), -s);
+            const float p = fmaf(dl, a.invbin, pos);  // from bin `start`
+            const bool ok = p > glo && p < ghi;
+            const int i = (int)floorf(p);
+            const int g = max(0, min(start + i, a.Nfft - 2));
+            const float2 v0 = row[g], v1 = row[g + 1];
+            const float f = p - (float)i;
+            const float vr = ok ? fmaf(f, v1.x - v0.x, v0.x) : 0.f;
+            const float vi = ok ? fmaf(f, v1.y - v0.y, v0.y) : 0.f;
+            const float ph = __builtin_amdgcn_fractf(fmaf(dl, kap, psi));
+            const float sn = __builtin_amdgcn_sinf(ph);
+            const float cs = __builtin_amdgcn_cosf(ph);
+            accr[j] = fmaf(vr, cs, fmaf(-vi, sn, accr[j]));
+            acci[j] = fmaf(vr, sn, fmaf(vi, cs, acci[j]));
+        }
+    }
+
+    // All pulses in [nbeg, nend).
+    template <class Pos>
+    __device__ __forceinline__ void run(const BpArgs &a, Lds &L, float *,
+                                        const float2 *__restrict__ prof, const Pos &pos,
+                                        const double *__restrict__ r0,
+                                        const double *__restrict__ f0, int nbeg, int nend) {
+        for (int n0 = nbeg; n0 < nend;) {
+            stage(a, L, prof, pos, r0, f0, n0, min(CH, nend - n0));
+            const int nc = L.nc;
+            if (__builtin_amdgcn_readfirstlane(L.fast)) {
+                for (int c = 0; c < nc; c++) pulse<false>(a, L, c);
+            } else {
+                for (int c = 0; c < nc; c++) {
+                    const int mode = __builtin_amdgcn_readfirstlane(L.pI[c].w);
+                    if (mode == kPulseFast) pulse<false>(a, L, c);
+                    else if (mode == kPulseGated) pulse<true>(a, L, c);
+                    else pulse_direct(a, L, c, prof + (size_t)(n0 + c) * a.Nfft);
+                }
+            }
+            n0 += nc;
         }
     }
 };

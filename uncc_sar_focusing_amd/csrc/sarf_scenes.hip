@@ -31,14 +31,18 @@ struct SceneDev {
     const float2 *prof;
     const double *ant, *r0, *f0;
     float2 *img;
-    int shape;  // mixed batches: index of the scene's tile in kMixedIds
+    int shape;  // mixed batches: index of the scene's tile in kMixedIds, 3 for
+                // tile 15 with windows wider than kBpCapX
 };
 
-// Tiles of a mixed batch (all 2048 pixels, lanes along x) and their engines.
+// Tiles of a mixed batch (all 2048 pixels, lanes along x) and their engines,
+// the ones sarf_backproject runs.  Four workgroups per CU: with five, the
+// engines behind a call spilled in their loops (16 scenes 5.5 -> 6.1 ms).
 constexpr int kMixedIds[3] = {15, 16, 13};
-using MixedT0 = BpTile<256, 8, true>;
+using MixedT0 = BpTileU<256, 8, true>;
 using MixedT1 = BpTile<128, 8, true>;
 using MixedT2 = BpTile<64, 8, true>;
+using MixedT3 = BpTile<256, 8, true>;
 // One engine's LDS (staging and per-column terms); a mixed kernel holds
 // the union, no more than the largest engine alone.
 template <class Tile>
@@ -50,8 +54,9 @@ union MixedLds {
     EngineLds<MixedT0> e0;
     EngineLds<MixedT1> e1;
     EngineLds<MixedT2> e2;
+    EngineLds<MixedT3> e3;
 };
-// the three engines share one occupancy target
+// the engines share one occupancy target
 static_assert(bp_waves_per_eu<256, 8, true>() == bp_waves_per_eu<128, 8, true>() &&
                   bp_waves_per_eu<128, 8, true>() == bp_waves_per_eu<64, 8, true>(),
               "mixed tiles: one waves-per-EU target");
@@ -60,14 +65,11 @@ __global__ void reset_counter(unsigned int *c) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0u;
 }
 
-template <int TY, int PX, bool XL>
-__global__ __launch_bounds__(kBpThreads) __attribute__((amdgpu_waves_per_eu(bp_waves_per_eu<TY, PX, XL>())))
-void bp_scenes(const SceneDev *__restrict__ scenes,
-                                                        const int2 *__restrict__ items,
-                                                        int nitems,
-                                                        unsigned int *__restrict__ counter) {
-    __shared__ typename BpTile<TY, PX, XL>::Lds L;
-    __shared__ __align__(16) float fx[BpTile<TY, PX, XL>::kFx];
+template <class Tile, int WAVES>
+__global__ __launch_bounds__(kBpThreads) __attribute__((amdgpu_waves_per_eu(WAVES)))
+void bp_scenes(const SceneDev *__restrict__ scenes, const int2 *__restrict__ items, int nitems,
+               unsigned int *__restrict__ counter) {
+    __shared__ EngineLds<Tile> E;
     __shared__ int sItem;
     for (;;) {
         __syncthreads();  // previous item done with sItem and L
@@ -78,11 +80,11 @@ void bp_scenes(const SceneDev *__restrict__ scenes,
         const int2 w = items[it];
         const SceneDev &S = scenes[w.x];
         const BpArgs a = S.a;
-        BpTile<TY, PX, XL> T;
+        Tile T;
         T.init(a, w.y);
-        T.run(a, L, fx, S.prof, PlainPos{S.ant}, S.r0, S.f0, 0, a.Np);
+        T.run(a, E.L, E.fx, S.prof, PlainPos{S.ant}, S.r0, S.f0, 0, a.Np);
 #pragma unroll
-        for (int j = 0; j < PX; j++) {
+        for (int j = 0; j < Tile::kPx; j++) {
             int x, y;
             if (T.pixel(j, x, y, a)) S.img[(size_t)x * a.Ny + y] = make_float2(T.accr[j], T.acci[j]);
         }
@@ -124,7 +126,8 @@ __attribute__((amdgpu_waves_per_eu(bp_waves_per_eu<256, 8, true>()))) void bp_sc
         switch (S.shape) {
             case 0: scene_item<MixedT0>(S, w.y, L.e0.L, L.e0.fx); break;
             case 1: scene_item<MixedT1>(S, w.y, L.e1.L, L.e1.fx); break;
-            default: scene_item<MixedT2>(S, w.y, L.e2.L, L.e2.fx); break;
+            case 2: scene_item<MixedT2>(S, w.y, L.e2.L, L.e2.fx); break;
+            default: scene_item<MixedT3>(S, w.y, L.e3.L, L.e3.fx); break;
         }
     }
 }
@@ -133,8 +136,8 @@ template <int TY, int PX, bool XL = false>
 void launch_scenes_t(int grid, const SceneDev *sc, const int2 *items, int nitems,
                      unsigned int *counter, hipStream_t s) {
     hipLaunchKernelGGL(reset_counter, dim3(1), dim3(64), 0, s, counter);
-    hipLaunchKernelGGL((bp_scenes<TY, PX, XL>), dim3(grid), dim3(kBpThreads), 0, s, sc, items,
-                       nitems, counter);
+    hipLaunchKernelGGL((bp_scenes<BpTile<TY, PX, XL>, bp_waves_per_eu<TY, PX, XL>()>), dim3(grid),
+                       dim3(kBpThreads), 0, s, sc, items, nitems, counter);
 }
 
 // Tile ids compiled for batches (at most 8 pixels per lane).
@@ -246,6 +249,7 @@ extern "C" int sarf_bp_scenes(sarf_ctx *ctx, int nscenes, const sarf_scene *scen
         BpArgs a{};
         const int rc = bp_fill_args(ctx, &d, st, &a);
         if (rc != SARF_OK) return fail(rc, "sarf_bp_scenes: scene %d: %s", i, sarf_last_error());
+        if (mixed && st == 15 && !a.narrow) shape = 3;
         host[i] = SceneDev{a, (const float2 *)c.prof, c.ant, c.r0, c.f0, (float2 *)c.img, shape};
         const int nt = a.tiles_x * a.tiles_y;
         for (int t = 0; t < nt; t++) items.push_back(Item{i, t, (double)c.Np * tx * ty});
@@ -296,7 +300,18 @@ extern "C" int sarf_bp_scenes(sarf_ctx *ctx, int nscenes, const sarf_scene *scen
         case 12: launch_scenes_t<64, 4, true>(grid, dsc, ditems, nit, counter, s); break;
         case 13: launch_scenes_t<64, 8, true>(grid, dsc, ditems, nit, counter, s); break;
         case 14: launch_scenes_t<32, 8, true>(grid, dsc, ditems, nit, counter, s); break;
-        case 15: launch_scenes_t<256, 8, true>(grid, dsc, ditems, nit, counter, s); break;
+        case 15: {
+            bool narrow = true;
+            for (const SceneDev &h : host) narrow = narrow && h.a.narrow;
+            if (!narrow) {
+                launch_scenes_t<256, 8, true>(grid, dsc, ditems, nit, counter, s);
+                break;
+            }
+            hipLaunchKernelGGL(reset_counter, dim3(1), dim3(64), 0, s, counter);
+            hipLaunchKernelGGL((bp_scenes<MixedT0, kBpWavesU>), dim3(std::min(nit, kBpWavesU * cus)),
+                               dim3(kBpThreads), 0, s, dsc, ditems, nit, counter);
+            break;
+        }
         case 16: launch_scenes_t<128, 8, true>(grid, dsc, ditems, nit, counter, s); break;
     }
     SARF_HIP(hipGetLastError());
