@@ -483,11 +483,19 @@ bool split_head_tail(const sarf_ctx *ctx, int tile, int ntiles, int Np) {
     return (long)ntiles >= 2 * resident && Np >= 64;
 }
 
-int default_splits(const sarf_ctx *ctx, int tile, int ntiles, int Np) {
+// Where that leaves CUs without a workgroup (the smallest images), on down to
+// 4 pulses per group: a lone workgroup's time is its chain of LDS and memory
+// latencies per pulse (128^2 x 117 pulses, 8 tiles: 4 groups 27.8 us, 8 groups
+// 20.5, 16 groups 15.8, 32 groups 16.1).  Not for the image a gradient is taken
+// of, which is rounded as it always was.
+int default_splits(const sarf_ctx *ctx, int tile, int ntiles, int Np, bool for_gradient) {
     if (split_head_tail(ctx, tile, ntiles, Np)) return 3;
     int splits = 1;
-    const long want = 64L * (ctx->cu_count > 0 ? ctx->cu_count : 256);
+    const long cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    const long want = 64L * cus;
     while (splits < 32 && (long)ntiles * splits < want && Np / (2 * splits) >= 16) splits *= 2;
+    while (!for_gradient && splits < 32 && (long)ntiles * splits < cus && Np / (2 * splits) >= 4)
+        splits *= 2;
     return splits;
 }
 
@@ -514,7 +522,8 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
     int tx = 0, ty = 0;
     const int tid = bp_tile_shape(tile, &tx, &ty);
     const int ntiles = a.tiles_x * a.tiles_y;
-    if (splits <= 0) splits = default_splits(ctx, tile, ntiles, d->Np);
+    if (splits <= 0)
+        splits = default_splits(ctx, tile, ntiles, d->Np, (d->flags & SARF_BP_FOR_GRADIENT) != 0);
     splits = std::max(1, std::min(splits, d->Np));
     const long npix = (long)d->Nx * d->Ny;
     float2 *o = (float2 *)img;
@@ -655,7 +664,9 @@ int launch_backproject_ext(sarf_ctx *ctx, const sarf_bp_desc *d, const void *pro
         if (!bp_tile_shape(tile, &tx, &ty))
             return fail(SARF_ERR_INVALID, "backproject: unknown tile id %d", tile);
         const int ntiles = ((d->Nx + tx - 1) / tx) * ((d->Ny + ty - 1) / ty);
-        if (splits <= 0) splits = default_splits(ctx, tile, ntiles, d->Np);
+        if (splits <= 0)
+            splits = default_splits(ctx, tile, ntiles, d->Np,
+                                    (d->flags & SARF_BP_FOR_GRADIENT) != 0);
         const size_t img_bytes = sizeof(float2) * (size_t)d->Nx * d->Ny;
         while (splits > 1 &&
                img_bytes * split_partials(splits, split_tail(ctx, tile, ntiles, d->Np, splits)) >
@@ -754,7 +765,7 @@ extern "C" int sarf_autotune(sarf_ctx *ctx, const sarf_bp_desc *d, const void *p
         int tx = 0, ty = 0;
         bp_tile_shape(best_tile, &tx, &ty);
         const int ntiles = ((d->Nx + tx - 1) / tx) * ((d->Ny + ty - 1) / ty);
-        best_split = std::max(1, std::min(default_splits(ctx, best_tile, ntiles, d->Np), d->Np));
+        best_split = std::max(1, std::min(default_splits(ctx, best_tile, ntiles, d->Np, false), d->Np));
     }
     // leave the image made with the chosen shape
     SARF_TRY(launch_mixed_shape(ctx, &dd, best_tile, best_split, prof, ant, r0, f0, img, s));
