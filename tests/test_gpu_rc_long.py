@@ -51,6 +51,19 @@ def test_other_lengths_f32(ctx, nfft):
         _check(ctx, Np, K, nfft, np.complex64, False, True, 2e-6)
 
 
+# the convolution length follows N + K - 1: the last K of one power of two and the
+# first of the next, in the register-resident and the global-memory form
+@pytest.mark.parametrize("nfft,K,dtype", [
+    (3000, 1097, np.complex64), (3000, 1098, np.complex64), (37, 28, np.complex64),
+    (37, 29, np.complex64), (5000, 3193, np.complex64), (8191, 2, np.complex64),
+    (8191, 1, np.complex64), (9000, 7385, np.complex64), (9000, 7386, np.complex64),
+    (1000, 25, np.complex128), (1000, 26, np.complex128), (3, 1, np.complex128)])
+def test_convolution_length(ctx, nfft, K, dtype):
+    single = dtype == np.complex64
+    for Np in (1, 6):
+        _check(ctx, Np, K, nfft, dtype, True, single, 2e-6 if single else 1e-14)
+
+
 # 128 MB of rows a slab: 256 pulses of 2^16 bins, 128 of 2^17 (three passes),
 # 512 of a Bluestein length of 2^15
 @pytest.mark.parametrize("Np,K,nfft", [(259, 30, 65536), (130, 500, 131072), (515, 77, 16001)])

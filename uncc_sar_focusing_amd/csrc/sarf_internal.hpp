@@ -62,7 +62,8 @@ struct sarf_ctx {
     std::map<long, float2 *> tw32;
     std::map<long, double2 *> tw64;
     // Bluestein tables, one allocation per key: range compression of
-    // length N in FP32 (key N) or FP64 (key -N); PGA rows of length N
+    // length N through M = 2^L in FP32 (key L 2^24 + N) or FP64 (its negative);
+    // PGA rows of length N
     // (key sarf::kPgaTableKey + N)
     std::map<long, void *> rc_blue;
     // named scratch buffers (partial images, reductions, staging); a buffer
@@ -125,8 +126,8 @@ int twiddles_any_f64(sarf_ctx *ctx, long n, const double2 **out);
 int ilog2_exact(long n);  // log2 if n is a power of two, else -1
 
 // Bluestein chirp and kernel spectrum of a length-N DFT with transform
-// length M = 2^L >= 2N - 1, in FP64: c_k = e^{+j pi k^2 / N} (k < N) and
-// C = FFT_M(h), h_d = conj(c_d) for d < N, h_{M-d} = conj(c_d) for 0 < d < N.
+// length M = 2^L > N, in FP64: c_k = e^{+j pi k^2 / N} (k < N) and C = FFT_M(h),
+// h_d = conj(c_d) for d < N, h_{M-d} = conj(c_d) for 0 < d < N as far as M > N + d.
 void bluestein_f64(int N, int L, std::vector<double> &cr, std::vector<double> &ci,
                    std::vector<double> &hr, std::vector<double> &hi);
 

@@ -98,6 +98,9 @@ __device__ __forceinline__ void rc_lds_body(const Jobs &J, int ngroups,
     const int tid = threadIdx.x;
     const int lp = tid / T, j = tid % T;
     float2 *L = lds + lp * PADN;
+    // 1/N and the ramp of each pulse, formed by one lane (by every lane, the
+    // FP64 sine and cosine were a tenth of the kernel)
+    __shared__ float2 ramp[P];
 
     // Sample row i of pulse n (sample k = j + i*T) as pass 0 consumes it:
     // zero padding (k >= K is never loaded), taper, fftshift fold (-1)^k.
@@ -147,6 +150,10 @@ __device__ __forceinline__ void rc_lds_body(const Jobs &J, int ngroups,
         // which would hold them in registers across iterations.
         int jj = j;
         __asm__ volatile("" : "+v"(jj));
+        if ((job.flags & SARF_RC_RAMP) && active && jj == 0) {
+            const double a = -4.0 * kPi * job.f0[n] * job.r0[n] / kClight;
+            ramp[lp] = make_float2((float)(cos(a) / N), (float)(sin(a) / N));
+        }
         float2 v[16];
         // ---- pass 0: registers -> LDS, radix R0, Ns = 1 (no twiddles) ------
         // lane input r of butterfly b is sample row i = b + r * NB0
@@ -208,9 +215,8 @@ __device__ __forceinline__ void rc_lds_body(const Jobs &J, int ngroups,
                 // Ns = N/16: output index j + r*N/16, coalesced per r
                 float sr = 1.0f / N, si = 0.0f;
                 if (job.flags & SARF_RC_RAMP) {
-                    double a = -4.0 * kPi * job.f0[n] * job.r0[n] / kClight;
-                    sr = (float)(cos(a) / N);
-                    si = (float)(sin(a) / N);
+                    sr = ramp[lp].x;
+                    si = ramp[lp].y;
                 }
                 float2 *dst = job.prof + (size_t)n * N;
 #pragma unroll
@@ -456,7 +462,8 @@ __global__ __launch_bounds__(pass_threads<T2>()) void rc_pass(PassArgs<T2> p) {
 // Nfft not a power of two, up to 8192 (e.g. the reference's default
 // N_fft = K, charlotte_sar_api.hpp:173): Bluestein's identity
 // k m = (k^2 + m^2 - (m - k)^2) / 2 turns the length-N inverse DFT into a
-// circular convolution of length M = 2^ceil(log2(2N - 1)):
+// circular convolution of length M = 2^ceil(log2(N + K - 1)) (the K samples
+// meet chirp offsets -(K - 1) .. N - 1):
 //   X_m = c_m sum_k (x_k c_k) conj(c_{m-k}),   c_k = e^{+j pi k^2 / N},
 // formed per pulse by two register-resident radix-16 transforms of length M
 // (sarf_fft.hpp): the forward transform of a_k = x_k c_k as conj(ifft(conj)),
@@ -467,7 +474,8 @@ __global__ __launch_bounds__(pass_threads<T2>()) void rc_pass(PassArgs<T2> p) {
 // of M/16 lanes per pulse, rows packed to >= 256 lanes per workgroup.
 // ---------------------------------------------------------------------------
 template <int LOG2M>
-__global__ __launch_bounds__(fft::group_threads(LOG2M)) void rc_bluestein(
+__global__ __launch_bounds__(fft::group_threads(LOG2M))
+__attribute__((amdgpu_waves_per_eu(LOG2M <= 13 ? 4 : 1))) void rc_bluestein(
     const float2 *__restrict__ ph, int K, int N, int Np, int flags,
     const float *__restrict__ taper, const double *__restrict__ f0,
     const double *__restrict__ r0, const float2 *__restrict__ chirp,
@@ -480,6 +488,16 @@ __global__ __launch_bounds__(fft::group_threads(LOG2M)) void rc_bluestein(
     const int n = blockIdx.x * P + lp;
     const bool active = n < Np;
     float2 *Lr = lds + lp * PAD;
+    __shared__ float2 ramp[P];  // scale and ramp of each pulse, formed by one lane
+    if (active && j == 0) {
+        double sr = 1.0 / ((double)M * N), si = 0.0;
+        if (flags & SARF_RC_RAMP) {
+            const double ang = -4.0 * kPi * f0[n] * r0[n] / kClight;
+            sr = cos(ang) / ((double)M * N);
+            si = sin(ang) / ((double)M * N);
+        }
+        ramp[lp] = make_float2((float)sr, (float)si);
+    }
     const float2 *x = ph + (size_t)(active ? n : 0) * K;
     float2 v[16];
 #pragma unroll
@@ -505,13 +523,7 @@ __global__ __launch_bounds__(fft::group_threads(LOG2M)) void rc_bluestein(
     fft::to_input_order<LOG2M>(u, v);
     fft::ifft_regs<LOG2M>(v, Lr, j, twM);  // v[r] = M (a * conj c)_{j + r*T}
     if (!active) return;
-    double sr = 1.0 / ((double)M * N), si = 0.0;
-    if (flags & SARF_RC_RAMP) {
-        const double ang = -4.0 * kPi * f0[n] * r0[n] / kClight;
-        sr = cos(ang) / ((double)M * N);
-        si = sin(ang) / ((double)M * N);
-    }
-    const float fr = (float)sr, fi = (float)si;
+    const float fr = ramp[lp].x, fi = ramp[lp].y;
     const int half = (N + 1) / 2;
     float2 *out = prof + (size_t)n * N;
 #pragma unroll
@@ -599,7 +611,7 @@ int launch_jobs(const sarf_ctx *ctx, int rows, const RcJob *jobs, int njobs, int
 // Bluestein chirp and kernel spectrum of a length-N DFT with transform
 // length M = 2^L, in FP64: c_k = e^{+j pi k^2 / N} (k < N; the phase from the
 // exact k^2 mod 2N) and C = FFT_M(h) with h_d = conj(c_d) for d < N,
-// h_{M-d} = conj(c_d) for 0 < d < N, zero between (iterative radix 2 over
+// h_{M-d} = conj(c_d) for 0 < d < N as far as M > N + d, zero between (iterative radix 2 over
 // directly evaluated twiddles).
 void bluestein_f64(int N, int L, std::vector<double> &cr, std::vector<double> &ci,
                    std::vector<double> &hr, std::vector<double> &hi) {
@@ -617,7 +629,7 @@ void bluestein_f64(int N, int L, std::vector<double> &cr, std::vector<double> &c
     for (int d = 0; d < N; d++) {
         hr[d] = cr[d];
         hi[d] = -ci[d];
-        if (d > 0) {
+        if (d > 0 && d <= M - N) {
             hr[M - d] = cr[d];
             hi[M - d] = -ci[d];
         }
@@ -655,13 +667,24 @@ void bluestein_f64(int N, int L, std::vector<double> &cr, std::vector<double> &c
 
 namespace {
 
+// log2 of the transform length that convolves K samples with the chirp of a
+// length-N transform without wrapping into its N outputs: the smallest power of
+// two >= N + K - 1 (with 2 N - 1 whatever K, 1237 pulses of 731 samples to 3000
+// bins took 64 us for the 32 they take now).
+int bluestein_log2(int N, int K, int least) {
+    int L = least;
+    while ((1L << L) < (long)N + K - 1) L++;
+    return L;
+}
+
 // Bluestein tables of a length-N inverse DFT with transform length M = 2^L
-// (cached per N and precision in the context): chirp (N) and C (M) of
+// (cached per N, M and precision in the context): chirp (N) and C (M) of
 // bluestein_f64, rounded once to T2.  One allocation [chirp (N) | C (M)].
 template <typename T2>
 int bluestein_tables(sarf_ctx *ctx, int N, int L, const T2 **chirp, const T2 **C) {
     const int M = 1 << L;
-    const long key = sizeof(T2) == sizeof(double2) ? -(long)N : (long)N;
+    const long id = (long)L << 24 | N;  // N <= 2^20
+    const long key = sizeof(T2) == sizeof(double2) ? -id : id;
     std::lock_guard<std::mutex> lk(ctx->mu);
     auto it = ctx->rc_blue.find(key);
     if (it == ctx->rc_blue.end()) {
@@ -862,9 +885,8 @@ int launch_range_compress(sarf_ctx *ctx, const sarf_rc_desc *d, const void *ph,
     const bool f64 = (d->flags & SARF_RC_F64) != 0;
     if (log2n < 0 && !f64 && d->Nfft <= kBluesteinMaxN) {
         // not a power of two: Bluestein through two register-resident
-        // transforms of length M = 2^ceil(log2(2N - 1))
-        int L = 5;
-        while ((1 << L) < 2 * d->Nfft - 1) L++;
+        // transforms of length M
+        const int L = bluestein_log2(d->Nfft, d->K, 5);
         const float2 *chirp = nullptr, *C = nullptr, *tw = nullptr;
         SARF_TRY(bluestein_tables<float2>(ctx, d->Nfft, L, &chirp, &C));
         SARF_TRY(twiddles_f32(ctx, L, &tw));
@@ -892,8 +914,7 @@ int launch_range_compress(sarf_ctx *ctx, const sarf_rc_desc *d, const void *ph,
         if (d->Nfft > kBluesteinGlobalMaxN)
             return fail(SARF_ERR_UNSUPPORTED, "range_compress: Nfft=%d (lengths that are not a "
                         "power of two go up to %d)", d->Nfft, kBluesteinGlobalMaxN);
-        int L = 1;
-        while ((1 << L) < 2 * d->Nfft - 1) L++;
+        const int L = bluestein_log2(d->Nfft, d->K, 1);
         if (f64)
             return launch_bluestein_global<double2>(ctx, d, L, (const double2 *)ph, taper, f0, r0,
                                                     (double2 *)prof, s);
