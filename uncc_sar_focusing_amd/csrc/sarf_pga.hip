@@ -434,14 +434,13 @@ __device__ __forceinline__ bool integrate_body(const PgaImage &p, int it, const 
 }
 
 // Short rows (M <= 512): one workgroup of kThreads per row, the row in LDS
-// (dynamic, M float2), radix-2 transforms -- more lanes per row than the
+// (buf, M float2), radix-2 transforms -- more lanes per row than the
 // register-resident kernels give, so lower latency at these lengths.
 // Step 3 for row y:
 // G[y][k] = e^{-j 2 pi k (s - fl)/N} DFT_x( mask[(x + s) mod N] At[y][x] )_k,
 // fl = floor(N/2): the shift by s, the mask and ifftshift as one remap.
-__device__ void row_dft_lds_body(const PgaImage &p, int y) {
+__device__ __forceinline__ void row_dft_lds_body(const PgaImage &p, int y, float2 *buf) {
     if (stopped(p)) return;
-    extern __shared__ float2 buf[];
     const int N = p.Nx, L = p.L, M = 1 << L;
     const int s = p.shift[y];
     const float2 *row = p.At + (size_t)y * N;
@@ -474,9 +473,8 @@ __device__ void row_dft_lds_body(const PgaImage &p, int y) {
 // which is the circular convolution At[y] (*)_N h, h = IDFT_N(e^{-j phi}):
 // the row zero-padded to M, times B = FFT_M(h extended over -(N-1)..N-1)
 // (apply_spectrum_body), back, and the bins N-1 .. 2N-2 are the result.
-__device__ void row_apply_lds_body(const PgaImage &p, int y) {
+__device__ __forceinline__ void row_apply_lds_body(const PgaImage &p, int y, float2 *buf) {
     if (stopped(p)) return;
-    extern __shared__ float2 buf[];
     const int N = p.Nx, L = p.L, M = 1 << L;
     float2 *row = p.At + (size_t)y * N;
     for (int x = threadIdx.x; x < M; x += kThreads)
@@ -865,8 +863,9 @@ __global__ __launch_bounds__(kSpecThreads) void k1_integrate(PgaImage p, int it)
     integrate_fused_body(p, it, Lr, phid, eph);
 }
 __global__ __launch_bounds__(kThreads) void k1_rows_lds(PgaImage p, int apply) {
-    if (apply) row_apply_lds_body(p, blockIdx.x);
-    else row_dft_lds_body(p, blockIdx.x);
+    extern __shared__ float2 buf[];
+    if (apply) row_apply_lds_body(p, blockIdx.x, buf);
+    else row_dft_lds_body(p, blockIdx.x, buf);
 }
 template <int LOG2M>
 __global__ __launch_bounds__(fft::group_threads(LOG2M)) void k1_rows(PgaImage p, int apply) {
@@ -959,8 +958,9 @@ __global__ __launch_bounds__(kThreads) void kb_rows_lds(PgaBatchDev b, int g0, i
     const int *ids = b.grp + g0, *off = ids + m;
     const int k = owner(off, m, blockIdx.x);
     const PgaImage p = b.img[ids[k]];
-    if (apply) row_apply_lds_body(p, blockIdx.x - off[k]);
-    else row_dft_lds_body(p, blockIdx.x - off[k]);
+    extern __shared__ float2 buf[];
+    if (apply) row_apply_lds_body(p, blockIdx.x - off[k], buf);
+    else row_dft_lds_body(p, blockIdx.x - off[k], buf);
 }
 // M <= 4096: capped at 128 VGPRs for four waves per SIMD (the LDS allows four
 // blocks per CU); the few spills cost less than the lost occupancy (64 uneven
@@ -976,6 +976,35 @@ __attribute__((amdgpu_waves_per_eu(LOG2M <= 12 ? 4 : 1))) void kb_rows(PgaBatchD
     __shared__ float2 lds[row_lds_elems<LOG2M>()];
     if (apply) row_apply_body<LOG2M>(p, blockIdx.x - off[k], lds);
     else row_dft_body<LOG2M>(p, blockIdx.x - off[k], lds);
+}
+
+// Row step of every image with M <= 4096 in one launch (all of them
+// workgroups of kThreads): per transform length the images of kb_rows or
+// kb_rows_lds, longest first.  grp[r0 .. r0 + m) are the images' ids, grp[r0 + m
+// .. r0 + 2m] their block offsets.  As a launch per length each length ran
+// alone, a few rounds of workgroups with a tail of its own (12 images of 150 to
+// 1000 a side, three lengths: 27 + 15 + 12 us a step; 39 to 47 merged, five
+// iterations 802 -> 685 us; bound by FP32 issue, about 30 us of it).
+constexpr int kMergedMaxL = 12;
+static_assert(fft::group_threads(10) == kThreads && fft::group_threads(kMergedMaxL) == kThreads,
+              "one workgroup size");
+template <bool APPLY>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void kb_rows_merged(
+    PgaBatchDev b, int r0, int m) {
+    const int *ids = b.grp + r0, *off = ids + m;
+    const int k = owner(off, m, blockIdx.x);
+    const PgaImage p = b.img[ids[k]];
+    const int blk = blockIdx.x - off[k];
+    __shared__ float2 lds[row_lds_elems<kMergedMaxL>()];
+    static_assert(row_lds_elems<10>() <= row_lds_elems<kMergedMaxL>() &&
+                      row_lds_elems<11>() <= row_lds_elems<kMergedMaxL>(),
+                  "one LDS block");
+    switch (p.L) {
+        case 12: APPLY ? row_apply_body<12>(p, blk, lds) : row_dft_body<12>(p, blk, lds); break;
+        case 11: APPLY ? row_apply_body<11>(p, blk, lds) : row_dft_body<11>(p, blk, lds); break;
+        case 10: APPLY ? row_apply_body<10>(p, blk, lds) : row_dft_body<10>(p, blk, lds); break;
+        default: APPLY ? row_apply_lds_body(p, blk, lds) : row_dft_lds_body(p, blk, lds);
+    }
 }
 
 // ---------------------------------------------------------------- host
@@ -1215,6 +1244,27 @@ extern "C" int sarf_pga_scenes(sarf_ctx *ctx, int nscenes, const sarf_pga_scene 
         }
         groups.push_back(g);
     }
+    // two or more transform lengths up to 2^kMergedMaxL: their row steps share
+    // launches
+    Group merged{0, (int)grp.size(), 0, 0};
+    {
+        std::vector<int> ids;
+        int lengths = 0;
+        for (auto g = groups.rbegin(); g != groups.rend(); ++g) {
+            if (g->L > kMergedMaxL) continue;
+            lengths++;
+            ids.insert(ids.end(), grp.begin() + g->g0, grp.begin() + g->g0 + g->m);
+        }
+        if (lengths > 1) {
+            merged.m = (int)ids.size();
+            grp.insert(grp.end(), ids.begin(), ids.end());
+            grp.push_back(0);
+            for (int id : ids) {
+                merged.blocks += row_blocks(host[id].L, host[id].Ny);
+                grp.push_back(merged.blocks);
+            }
+        }
+    }
     const size_t b_img = sizeof(PgaImage) * (size_t)n, b_off = sizeof(int) * off.size(),
                  b_grp = sizeof(int) * grp.size();
     const size_t b_desc = align256(b_img) + align256(b_off) + align256(b_grp);
@@ -1259,6 +1309,20 @@ extern "C" int sarf_pga_scenes(sarf_ctx *ctx, int nscenes, const sarf_pga_scene 
         SARF_HIP(hipStreamSynchronize(s));
     }
     const auto total = [&](int kind) { return off[(size_t)kind * (n + 1) + n]; };
+    const auto row_step = [&](int apply) -> int {
+        if (merged.m > 0) {
+            if (apply)
+                hipLaunchKernelGGL(kb_rows_merged<true>, dim3(merged.blocks), dim3(kThreads), 0, s,
+                                   b, merged.g0, merged.m);
+            else
+                hipLaunchKernelGGL(kb_rows_merged<false>, dim3(merged.blocks), dim3(kThreads), 0,
+                                   s, b, merged.g0, merged.m);
+        }
+        for (const Group &g : groups)
+            if (merged.m == 0 || g.L > kMergedMaxL)
+                SARF_TRY(kb_row_step(b, g.L, g.g0, g.m, g.blocks, apply, s));
+        return SARF_OK;
+    };
     if (iters == 0) hipLaunchKernelGGL(kb_setup, dim3(n), dim3(kThreads), 0, s, b);
     if (iters > 0) {
         hipLaunchKernelGGL(kb_transpose, dim3(total(kOffTranspose)), dim3(kThreads), 0, s, b, 1);
@@ -1266,11 +1330,11 @@ extern "C" int sarf_pga_scenes(sarf_ctx *ctx, int nscenes, const sarf_pga_scene 
             hipLaunchKernelGGL(kb_stats, dim3(total(kOffRows) + total(kOffColPartial)),
                                dim3(kThreads), 0, s, b, total(kOffRows));
             hipLaunchKernelGGL(kb_window, dim3(n), dim3(kIntThreads), 0, s, b, db_down);
-            for (const Group &g : groups) SARF_TRY(kb_row_step(b, g.L, g.g0, g.m, g.blocks, 0, s));
+            SARF_TRY(row_step(0));
             hipLaunchKernelGGL(kb_col_partial, dim3(total(kOffColPartial)), dim3(kThreads), 0, s,
                                b, 1);
             hipLaunchKernelGGL(kb_integrate, dim3(n), dim3(kSpecThreads), 0, s, b, it);
-            for (const Group &g : groups) SARF_TRY(kb_row_step(b, g.L, g.g0, g.m, g.blocks, 1, s));
+            SARF_TRY(row_step(1));
             SARF_HIP(hipGetLastError());
         }
         hipLaunchKernelGGL(kb_transpose, dim3(total(kOffTranspose)), dim3(kThreads), 0, s, b, 0);
