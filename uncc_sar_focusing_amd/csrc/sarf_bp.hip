@@ -557,7 +557,10 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
         case 2: launch_mixed_t<64, 4>(a, grid, p, ant, r0, f0, o, s); break;
         case 3: launch_mixed_t<64, 8>(a, grid, p, ant, r0, f0, o, s); break;
         case 4: launch_mixed_t<32, 8>(a, grid, p, ant, r0, f0, o, s); break;
-        case 5: launch_mixed_t<16, 4>(a, grid, p, ant, r0, f0, o, s); break;
+        case 5:
+            if (a.narrow) launch_mixed_t<16, 4, false, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
+            else launch_mixed_t<16, 4>(a, grid, p, ant, r0, f0, o, s);
+            break;
         case 6: launch_mixed_t<64, 16>(a, grid, p, ant, r0, f0, o, s); break;
         case 7: launch_mixed_t<32, 16>(a, grid, p, ant, r0, f0, o, s); break;
         case 11: launch_mixed_t<32, 4, true>(a, grid, p, ant, r0, f0, o, s); break;

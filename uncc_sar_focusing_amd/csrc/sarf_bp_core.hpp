@@ -65,9 +65,10 @@ static_assert(kBpChunk <= 64 && kBpCap % kBpThreads == 0, "staging layout");
 // Waves per SIMD the tile kernels are compiled for: 4 (<= 128 VGPRs) up to
 // 8 pixels per lane, except lanes-along-x tiles whose column terms take the
 // LDS past 40 KiB (3 workgroups per CU); the 16-pixel tiles need more
-// registers than that.  Tiles 13, 15 and 16 with the smaller windows: 5 (2048^2
+// registers than that.  Tiles 5, 13, 15 and 16 with the smaller windows: 5 (2048^2
 // at 0.05 m, 4096 pulses, tile 16 6.98 -> 6.74 ms, tile 13 7.23 -> 6.94; 1331
-// candidates at 512^2, 1024 pulses, tile 15 154.0 -> 150.2 ms, 153.7 with 4).
+// candidates at 512^2, 1024 pulses, tile 15 154.0 -> 150.2 ms, 153.7 with 4; 777 x
+// 603, 1237 pulses, tile 5 with range compression 367 -> 352 us).
 template <int TY, int PX, bool XL, int CAP = kBpCap>
 constexpr int bp_waves_per_eu() {
     return CAP < kBpCap ? 5 : PX > 8 ? 1 : (XL && (kBpThreads / TY) * PX > 32) ? 3 : 4;
