@@ -475,8 +475,12 @@ std::array<uint64_t, 8> tune_key(const sarf_bp_desc *d) { return tune_key(tune_g
 //   for 8 even groups and 8.04 ms unsplit, with 2 partial images instead of 8
 //   (a tail of 1/4, 1/6, 1/12 or 1/16 of the pulses measured 7.27-7.58 ms);
 // * even groups otherwise (few tiles: the groups are what fills the GPU),
-//   doubling until there are 64 workgroups per CU with at least 16 pulses
-//   per group (512^2 x 1024 pulses best at 16-32, 256^2 x 512 at 16).
+//   doubling until there are 16 workgroups per CU with at least 16 pulses
+//   per group.  Every group costs a partial image written and read again: 1024^2
+//   x 896 pulses (512 tiles) 361 us with 8 groups, 416 with 32; 1400 x 1000 x 600
+//   (693 tiles) 390 with 8, 503 with 32; 777 x 603 x 1237 (494 tiles) 304 with
+//   16, 323 with 32; 768^2 x 1000 (288) 232 with 16, 254 with 32; 512^2 x 1024
+//   (128) 118 with 16, 123 with 32; 256^2 x 512 (32) 34 with 16 to 32.
 
 bool split_head_tail(const sarf_ctx *ctx, int tile, int ntiles, int Np) {
     const long resident = (long)(ctx->cu_count > 0 ? ctx->cu_count : 256) * tile_waves_per_eu(tile);
@@ -486,13 +490,13 @@ bool split_head_tail(const sarf_ctx *ctx, int tile, int ntiles, int Np) {
 // Where that leaves CUs without a workgroup (the smallest images), on down to
 // 4 pulses per group: a lone workgroup's time is its chain of LDS and memory
 // latencies per pulse (128^2 x 117 pulses, 8 tiles: 4 groups 27.8 us, 8 groups
-// 20.5, 16 groups 15.8, 32 groups 16.1).  Not for the image a gradient is taken
-// of, which is rounded as it always was.
+// 20.5, 16 groups 15.8, 32 groups 16.1).  The image a gradient is taken of is
+// rounded as it always was: up to 64 workgroups per CU, 16 pulses or more.
 int default_splits(const sarf_ctx *ctx, int tile, int ntiles, int Np, bool for_gradient) {
     if (split_head_tail(ctx, tile, ntiles, Np)) return 3;
     int splits = 1;
     const long cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    const long want = 64L * cus;
+    const long want = (for_gradient ? 64L : 16L) * cus;
     while (splits < 32 && (long)ntiles * splits < want && Np / (2 * splits) >= 16) splits *= 2;
     while (!for_gradient && splits < 32 && (long)ntiles * splits < cus && Np / (2 * splits) >= 4)
         splits *= 2;
