@@ -200,9 +200,20 @@ int pinned_get(sarf_ctx *ctx, size_t bytes, char **out) {
     }
     if (!ctx->copier) {
         const unsigned hw = std::thread::hardware_concurrency();
-        ctx->copier = new HostCopier((int)std::max(1u, std::min(8u, hw ? hw : 1u)));
+        // parts of 256 KiB: a 2 MiB piece of an upload takes all threads
+        ctx->copier = new HostCopier((int)std::max(1u, std::min(8u, hw ? hw : 1u)), size_t(256) << 10);
     }
     *out = (char *)ctx->pinned;
+    return SARF_OK;
+}
+
+// The streams and events of the host-buffer path, kept for the life of the
+// context (creating and destroying them took a tenth of a 1024^2 call).
+static int focus_streams(sarf_ctx *ctx) {
+    for (hipStream_t *st : {&ctx->focus_up, &ctx->focus_run})
+        if (!*st) SARF_HIP(hipStreamCreateWithFlags(st, hipStreamNonBlocking));
+    for (hipEvent_t &e : ctx->focus_ev)
+        if (!e) SARF_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     return SARF_OK;
 }
 
@@ -275,6 +286,10 @@ int sarf_ctx_destroy(sarf_ctx *ctx) {
     for (auto &kv : ctx->scratch)
         if (kv.second.ptr) (void)hipFree(kv.second.ptr);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
+    for (hipEvent_t e : ctx->focus_ev)
+        if (e) (void)hipEventDestroy(e);
+    for (hipStream_t st : {ctx->focus_up, ctx->focus_run})
+        if (st) (void)hipStreamDestroy(st);
     delete ctx->copier;
     delete ctx;
     return SARF_OK;
@@ -325,10 +340,7 @@ int sarf_focus(sarf_ctx *ctx, const sarf_focus_desc *d, const float *ph, const d
     SARF_TRY(scratch_get(ctx, "focus.prof", prof_elems * csz, &dprof));
     SARF_TRY(scratch_get(ctx, "focus.img", img_elems * csz, &dimg));
     SARF_TRY(scratch_get(ctx, "focus.geo", sizeof(double) * 5 * d->Np, &dgeo));
-    double *dant = (double *)dgeo, *dr0 = dant + 3 * d->Np, *df0 = dr0 + d->Np;
-    SARF_HIP(hipMemcpy(dant, ant, sizeof(double) * 3 * d->Np, hipMemcpyHostToDevice));
-    SARF_HIP(hipMemcpy(dr0, r0, sizeof(double) * d->Np, hipMemcpyHostToDevice));
-    SARF_HIP(hipMemcpy(df0, f0, sizeof(double) * d->Np, hipMemcpyHostToDevice));
+    double *dant = (double *)dgeo, *dr0 = dant + 3 * (size_t)d->Np, *df0 = dr0 + d->Np;
     sarf_bp_desc bp{};
     bp.Nx = d->Nx; bp.Ny = d->Ny; bp.Nfft = d->Nfft; bp.Np = d->Np;
     bp.x0 = d->x0; bp.y0 = d->y0; bp.Wx = d->Wx; bp.Wy = d->Wy; bp.maxWr = d->maxWr;
@@ -352,6 +364,9 @@ int sarf_focus(sarf_ctx *ctx, const sarf_focus_desc *d, const float *ph, const d
     }
     if (f64) {
         // validation path: whole transfers, then RC and BP
+        SARF_HIP(hipMemcpy(dant, ant, sizeof(double) * 3 * d->Np, hipMemcpyHostToDevice));
+        SARF_HIP(hipMemcpy(dr0, r0, sizeof(double) * d->Np, hipMemcpyHostToDevice));
+        SARF_HIP(hipMemcpy(df0, f0, sizeof(double) * d->Np, hipMemcpyHostToDevice));
         std::vector<double> tmp(2 * ph_elems);
         for (size_t i = 0; i < 2 * ph_elems; i++) tmp[i] = ph[i];
         SARF_HIP(hipMemcpy(dph, tmp.data(), ph_elems * csz, hipMemcpyHostToDevice));
@@ -369,6 +384,10 @@ int sarf_focus(sarf_ctx *ctx, const sarf_focus_desc *d, const float *ph, const d
         // staging: the copies go straight from and to them.
         // The first group's upload is not overlapped with anything, so it is
         // kept short (an eighth of the pulses); the rest split evenly.
+        // Measured at 1024^2, 2048 pulses x 1024 samples (16 MiB up, 8 down):
+        // 1.72 ms with streams and events made per call, three synchronous
+        // geometry copies and one staging copy per group, 1.40 so; 4 groups
+        // instead of 3: 1.41, 8: 1.53 (fill and drain of each group).
         const int Gr = std::max(1, std::min(4, d->Np / 1024));
         const int G = Gr > 1 ? Gr + 1 : 1;
         const int first = G > 1 ? d->Np / 8 : d->Np;
@@ -386,29 +405,32 @@ int sarf_focus(sarf_ctx *ctx, const sarf_focus_desc *d, const float *ph, const d
         const bool ph_direct = host_pinned(ph, ph_elems * csz);
         const bool img_direct = host_pinned(img, img_bytes);
         char *pin = nullptr;
-        const size_t stage = (ph_direct ? 0 : 2 * slot) + (img_direct ? 0 : img_bytes);
-        if (stage > 0) SARF_TRY(pinned_get(ctx, stage, &pin));
-        char *pin_ph[2] = {nullptr, nullptr}, *pin_img = pin;
+        const size_t geo_bytes = sizeof(double) * 5 * (size_t)d->Np;
+        const size_t geo = (geo_bytes + 255) & ~(size_t)255;
+        SARF_TRY(pinned_get(ctx, geo + (ph_direct ? 0 : 2 * slot) + (img_direct ? 0 : img_bytes), &pin));
+        SARF_TRY(focus_streams(ctx));
+        // page-locked arrays may still be filled by work on the default stream
+        SARF_HIP(hipStreamSynchronize(nullptr));
+        char *pin_ph[2] = {nullptr, nullptr}, *pin_img = pin + geo;
         if (!ph_direct) {
-            pin_ph[0] = pin;
-            pin_ph[1] = pin + slot;
-            pin_img = pin + 2 * slot;
+            pin_ph[0] = pin + geo;
+            pin_ph[1] = pin_ph[0] + slot;
+            pin_img = pin_ph[1] + slot;
         }
         constexpr int kChunks = 4;
-        hipStream_t sc = nullptr, s = nullptr;
-        SARF_HIP(hipStreamCreateWithFlags(&sc, hipStreamNonBlocking));
-        if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {
-            (void)hipStreamDestroy(sc);
-            return fail(SARF_ERR_HIP, "sarf_focus: stream creation failed");
-        }
-        hipEvent_t copied[2] = {nullptr, nullptr}, dl[kChunks] = {};
+        const hipStream_t sc = ctx->focus_up, s = ctx->focus_run;
+        const hipEvent_t *copied = ctx->focus_ev, *dl = ctx->focus_ev + 2;
+        static_assert(2 + kChunks == sizeof(ctx->focus_ev) / sizeof(hipEvent_t), "events");
         int rc = SARF_OK;
-        for (hipEvent_t *e : {&copied[0], &copied[1]})
-            if (rc == SARF_OK && hipEventCreateWithFlags(e, hipEventDisableTiming) != hipSuccess)
-                rc = fail(SARF_ERR_HIP, "sarf_focus: event creation failed");
-        for (int c = 0; c < kChunks && rc == SARF_OK; c++)
-            if (hipEventCreateWithFlags(&dl[c], hipEventDisableTiming) != hipSuccess)
-                rc = fail(SARF_ERR_HIP, "sarf_focus: event creation failed");
+        {
+            // antenna, ranges and frequencies as one copy
+            double *h = (double *)pin;
+            std::memcpy(h, ant, sizeof(double) * 3 * (size_t)d->Np);
+            std::memcpy(h + 3 * (size_t)d->Np, r0, sizeof(double) * d->Np);
+            std::memcpy(h + 4 * (size_t)d->Np, f0, sizeof(double) * d->Np);
+            if (hipMemcpyAsync(dgeo, h, geo_bytes, hipMemcpyHostToDevice, s) != hipSuccess)
+                rc = fail(SARF_ERR_HIP, "sarf_focus: upload of the geometry failed");
+        }
         for (int g = 0; g < G && rc == SARF_OK; g++) {
             const int n0 = group_start(g), n1 = group_start(g + 1);
             const size_t off = (size_t)n0 * d->K, bytes = sizeof(float2) * (size_t)(n1 - n0) * d->K;
@@ -420,12 +442,23 @@ int sarf_focus(sarf_ctx *ctx, const sarf_focus_desc *d, const float *ph, const d
                     rc = fail(SARF_ERR_HIP, "sarf_focus: upload of group %d failed", g - 2);
                     break;
                 }
-                ctx->copier->copy(pin_ph[k], src, bytes);
-                src = pin_ph[k];
             }
-            if (hipMemcpyAsync((float2 *)dph + off, src, bytes, hipMemcpyHostToDevice, sc) !=
-                    hipSuccess ||
-                hipEventRecord(copied[k], sc) != hipSuccess ||
+            // in pieces of 2 MiB, each sent while the next is copied into the
+            // staging (pieces of 1 MiB: 1419 us instead of 1363 at 1024^2,
+            // 2048 pulses; 4 MiB: 1364, but no overlap in a smaller group)
+            const size_t piece = ph_direct ? bytes : size_t(2) << 20;
+            bool sent = true;
+            for (size_t o = 0; o < bytes && sent; o += piece) {
+                const size_t b = std::min(piece, bytes - o);
+                const char *from = (const char *)src + o;
+                if (!ph_direct) {
+                    ctx->copier->copy(pin_ph[k] + o, from, b);
+                    from = pin_ph[k] + o;
+                }
+                sent = hipMemcpyAsync((char *)((float2 *)dph + off) + o, from, b,
+                                      hipMemcpyHostToDevice, sc) == hipSuccess;
+            }
+            if (!sent || hipEventRecord(copied[k], sc) != hipSuccess ||
                 hipStreamWaitEvent(s, copied[k], 0) != hipSuccess) {
                 rc = fail(SARF_ERR_HIP, "sarf_focus: upload of pulses %d..%d failed", n0, n1);
                 break;
@@ -459,12 +492,6 @@ int sarf_focus(sarf_ctx *ctx, const sarf_focus_desc *d, const float *ph, const d
         }
         (void)hipStreamSynchronize(s);
         (void)hipStreamSynchronize(sc);
-        for (hipEvent_t e : copied)
-            if (e) (void)hipEventDestroy(e);
-        for (hipEvent_t e : dl)
-            if (e) (void)hipEventDestroy(e);
-        (void)hipStreamDestroy(s);
-        (void)hipStreamDestroy(sc);
         if (rc != SARF_OK) return rc;
     }
     if (f64) {

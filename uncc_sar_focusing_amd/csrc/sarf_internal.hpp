@@ -88,6 +88,10 @@ struct sarf_ctx {
     void *pinned = nullptr;
     size_t pinned_bytes = 0;
     sarf::HostCopier *copier = nullptr;
+    // its streams (upload, compute) and events (uploads of two staging slots,
+    // image chunks), created by the first call
+    hipStream_t focus_up = nullptr, focus_run = nullptr;
+    hipEvent_t focus_ev[6] = {};
 };
 
 namespace sarf {
