@@ -176,11 +176,26 @@ __device__ __forceinline__ int swizzle_tile(int b, int ntiles) {
     return (b & 7) * per + (b >> 3);
 }
 
+// LDS address of a position's bin without a conversion.  q = p - 1/32 (p: position
+// in bins, p >= 0) added to 2^19 + the window's first bin rounds to sixteenths of
+// a bin, the nearest sixteenth to p - 1/32 being floor(16 p) / 16, and the sum's
+// low mantissa bits are sixteen times the bin plus four bits of fraction: with
+// those masked off, the byte offset of the bin's 16 bytes.  The add and the mask
+// issue in about 2.4 cycles each per wave, v_cvt_i32_f32 and v_lshl_add_u32 in 4
+// (measured over 8 waves per SIMD: add, FMA, and 62-67 T lane operations/s, convert
+// and shift-add 38): 2048^2 x 4096 pulses with range compression 5.99 -> 5.82 ms.  At an integer p the sum may round to the bin below, whose
+// line meets the next one's there.
+constexpr float kBinShift = 0.03125f, kBinMagic = 524288.f;
+__device__ __forceinline__ int bin_bytes(float q, float magic) {
+    return __float_as_int(q + magic) & 0x7ff0;
+}
+
 // Bins of a tile's windows, staged by the whole workgroup: bin f of the
 // packed windows belongs to the last pulse c with offset <= f (pI.y), profile
 // bin pI.x + f - pI.y; the chunk's first profile is `base`.  In rounds of
 // kSlots bins per thread whose loads are all issued before any is consumed.
-template <int CH>
+// SHIFTED: intercepts for positions 1/32 bin below the true ones (kBinMagic).
+template <int CH, bool SHIFTED = false>
 __device__ __forceinline__ void fill_windows(float4 *win, const int4 *pI, int nc, int tot,
                                              const float2 *__restrict__ base, int Nfft) {
     const int tid = threadIdx.x;
@@ -213,7 +228,7 @@ __device__ __forceinline__ void fill_windows(float4 *win, const int4 *pI, int nc
             const int f = f0r + tid + k * kBpThreads;
             if (f < tot) {
                 const float dr = v1[k].x - v0[k].x, di = v1[k].y - v0[k].y;
-                const float fb = (float)wb[k];
+                const float fb = (float)wb[k] - (SHIFTED ? kBinShift : 0.f);
                 win[f] = make_float4(fmaf(-fb, dr, v0[k].x), fmaf(-fb, di, v0[k].y), dr, di);
             }
         }
@@ -567,7 +582,7 @@ struct BpLdsU {
     // (k: revolutions per metre; w: pixel spacing along the pixel axis)
     float4 qA[CH];  // -k u_l, k c2l, k c3l, psi_c
     float4 qB[CH];  // -k w u_p, k w e1, k w e2, k w^2 c2p
-    float4 qC[CH];  // k w^2 e3, bins per revolution, pos_c, LDS offset (bins, as int)
+    float4 qC[CH];  // k w^2 e3, bins per revolution, pos_c - kBinShift, kBinMagic + LDS offset (bins)
     int4 pI[CH];    // start bin, LDS offset, W, kPulse*
     float4 pA[CH];  // direct form: uh_x, uh_y, g0, g1
     float kap[CH];
@@ -585,6 +600,7 @@ struct BpTileU {
     static constexpr int CH = TL == 256 ? 64 : kBpChunk;
     static_assert(TL % 64 == 0 && PX % 2 == 0, "one range of pixel coordinates per wave");
     using Lds = BpLdsU<CH>;
+    static_assert(kBpCapX * 16 <= 0x8000, "bin_bytes");
     static constexpr int kFx = 4;  // no per-column terms (BpTile's interface)
     int ix0, iy0, ly, gx;
     double pcx, pcy, hx, hy;
@@ -651,7 +667,7 @@ struct BpTileU {
                                         (float)(kw * g1 * up * (1.0 - 3.0 * ul * ul)),
                                         (float)(kw * w * g0 * mp));
                 C = make_float4((float)(kw * w * g1 * ul * (1.0 - 3.0 * up * up)),
-                                (float)(a.binv / kap), (float)(posg - st), 0.f);
+                                (float)(a.binv / kap), (float)(posg - st - kBinShift), 0.f);
                 L.pA[tid] = make_float4((float)ah, (float)bh, (float)g0, (float)g1);
                 L.kap[tid] = (float)kap;
                 const bool inside = st >= 0.0 && st + wd <= a.Nfft && kap * ext <= 250.0;
@@ -675,7 +691,7 @@ struct BpTileU {
             const int nc = __popcll(__ballot(tid < cmax && incl <= kBpCapX));
             const bool slow = __ballot(tid < nc && mode != kPulseFast) != 0;
             if (tid < cmax) {
-                C.w = __int_as_float(incl - W);
+                C.w = kBinMagic + (float)(incl - W);
                 L.qC[tid] = C;
                 L.pI[tid] = make_int4(start, incl - W, W, mode);
             }
@@ -686,7 +702,7 @@ struct BpTileU {
             }
         }
         __syncthreads();
-        fill_windows<CH>(L.win, L.pI, L.nc, L.tot, prof + (size_t)n0 * a.Nfft, a.Nfft);
+        fill_windows<CH, true>(L.win, L.pI, L.nc, L.tot, prof + (size_t)n0 * a.Nfft, a.Nfft);
         __syncthreads();
     }
 
@@ -704,14 +720,14 @@ struct BpTileU {
             kA = fmaf(2.f * Pc, kB, kA);
         }
         const float by = __builtin_amdgcn_fractf(A.w + rev);
-        // window position at phase 0 of the reduced phase
+        // window position (less kBinShift) at phase 0 of the reduced phase
         const float bx = fmaf(C.y, rev - by, C.z);
-        const float4 *win = L.win + __float_as_int(C.w);
+        const char *win = (const char *)L.win;
         float glo = 0.f, ghi = 0.f, wmax = 0.f;
         if constexpr (GATED) {
             const int4 I = L.pI[c];
-            glo = (float)(-I.x);
-            ghi = (float)(a.Nfft - 1 - I.x);
+            glo = (float)(-I.x) - kBinShift;
+            ghi = (float)(a.Nfft - 1 - I.x) - kBinShift;
             wmax = (float)(I.z - 2);
         }
         // every window read of the pulse is issued before the first is used (left
@@ -724,7 +740,7 @@ struct BpTileU {
             ph[j] = fmaf(d, kA, fmaf(d * d, kB, by));
             p[j] = fmaf(ph[j], C.y, bx);
             // fast: the window has a bin of margin on each side, 1 <= p <= W - 2
-            w[j] = win[GATED ? (int)__builtin_amdgcn_fmed3f(p[j], 0.f, wmax) : (int)p[j]];
+            w[j] = *(const float4 *)(win + bin_bytes(GATED ? __builtin_amdgcn_fmed3f(p[j], 0.f, wmax) : p[j], C.w));
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -745,7 +761,7 @@ struct BpTileU {
                                                  const float2 *__restrict__ row) {
         const float4 A = L.pA[c];
         const int start = L.pI[c].x;
-        const float kap = L.kap[c], psi = L.qA[c].w, pos = L.qC[c].z;
+        const float kap = L.kap[c], psi = L.qA[c].w, pos = L.qC[c].z + kBinShift;
         const float ul = XL ? A.x : A.y, up = XL ? A.y : A.x;
         const float glo = (float)(-start), ghi = (float)(a.Nfft - 1 - start);
         // opaque, so that this path's per-pixel constants are not held in
