@@ -183,8 +183,9 @@ __device__ __forceinline__ int swizzle_tile(int b, int ntiles) {
 // those masked off, the byte offset of the bin's 16 bytes.  The add and the mask
 // issue in about 2.4 cycles each per wave, v_cvt_i32_f32 and v_lshl_add_u32 in 4
 // (measured over 8 waves per SIMD: add, FMA, and 62-67 T lane operations/s, convert
-// and shift-add 38): 2048^2 x 4096 pulses with range compression 5.99 -> 5.82 ms.  At an integer p the sum may round to the bin below, whose
-// line meets the next one's there.
+// and shift-add 38): 2048^2 x 4096 pulses with range compression 5.99 -> 5.82 ms.
+// At an integer p the sum may round to the bin below, whose line meets the next
+// one's there.
 constexpr float kBinShift = 0.03125f, kBinMagic = 524288.f;
 __device__ __forceinline__ int bin_bytes(float q, float magic) {
     return __float_as_int(q + magic) & 0x7ff0;
@@ -563,11 +564,13 @@ struct BpTile {
 // direct expansion over the profile in memory remains for pulses whose window
 // does not fit in LDS, that are so near that the cubic term along the pixel
 // axis (left out here) would show, or that have no carrier to speak of.
-// Bound by VALU issue: 97 instructions and 16 sines and cosines per 8 pixels and
-// pulse where BpTile takes 109 and 16.  It hides its LDS latencies only with
+// Bound by the LDS data path (0.86 of its rate at 2048^2) and VALU issue together:
+// 96 instructions and 16 sines and cosines per 8 pixels and pulse where BpTile
+// takes 109 and 16, and one 16-byte read per pixel and pulse.  It hides its LDS latencies only with
 // five waves per SIMD (kBpCapX is what five workgroups' LDS leaves; 96 VGPRs):
 // 2048^2 at 0.05 m, 4096 pulses, tile 15: BpTile 6.75 ms, this with four waves
-// 6.25, with five 5.85 (2.9 T pixel-pulses/s; six waves the same), and rel-L2
+// 6.25, with five 5.85 (six waves the same; 5.65 and 3.0 T pixel-pulses/s with the
+// addresses of bin_bytes), and rel-L2
 // against FP64 2.7e-6 -> 1.8e-6.  With 16 pixels per lane (107 instructions per
 // 8 pixels, 128 VGPRs, four waves) 6.29.  Only tile 15: tiles 16 and 13 keep
 // the rounding of BpTile, which is most of what their images are off by.
