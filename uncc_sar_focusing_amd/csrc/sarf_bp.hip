@@ -551,6 +551,11 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
         a.split_stride = npix;
     }
     const int grid = ntiles * splits;
+    // five waves per SIMD where there are workgroups for the fifth: 605 x 597, 94
+    // pulses (tile 16, 760 workgroups) with range compression 48.4 us with the
+    // kernel of four waves, which has registers to spare, 49.4 with five; 777 x
+    // 603 x 1237 (tile 5, 7904 workgroups) 367 with four, 351 with five
+    const bool five = a.narrow && grid > 4 * (ctx->cu_count > 0 ? ctx->cu_count : 256);
     const float2 *p = (const float2 *)prof;
     // Tile 15: BpTileU, except for the image a gradient is taken of, whose
     // rounding the adjoint kernel repeats, and where BpTile's larger windows
@@ -562,7 +567,7 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
         case 3: launch_mixed_t<64, 8>(a, grid, p, ant, r0, f0, o, s); break;
         case 4: launch_mixed_t<32, 8>(a, grid, p, ant, r0, f0, o, s); break;
         case 5:
-            if (a.narrow) launch_mixed_t<16, 4, false, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
+            if (five) launch_mixed_t<16, 4, false, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
             else launch_mixed_t<16, 4>(a, grid, p, ant, r0, f0, o, s);
             break;
         case 6: launch_mixed_t<64, 16>(a, grid, p, ant, r0, f0, o, s); break;
@@ -570,7 +575,7 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
         case 11: launch_mixed_t<32, 4, true>(a, grid, p, ant, r0, f0, o, s); break;
         case 12: launch_mixed_t<64, 4, true>(a, grid, p, ant, r0, f0, o, s); break;
         case 13:
-            if (a.narrow) launch_mixed_t<64, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
+            if (five) launch_mixed_t<64, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
             else launch_mixed_t<64, 8, true>(a, grid, p, ant, r0, f0, o, s);
             break;
         case 14: launch_mixed_t<32, 8, true>(a, grid, p, ant, r0, f0, o, s); break;
@@ -580,7 +585,7 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
             else launch_mixed_u<256, 8, true>(a, grid, p, ant, r0, f0, o, s);
             break;
         case 16:
-            if (a.narrow) launch_mixed_t<128, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
+            if (five) launch_mixed_t<128, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
             else launch_mixed_t<128, 8, true>(a, grid, p, ant, r0, f0, o, s);
             break;
         default: return fail(SARF_ERR_INVALID, "backproject: unknown tile id %d", tid);
