@@ -142,9 +142,10 @@ __device__ __forceinline__ double2 cis_rev64(double t) {
 }
 
 // Square root to within an ulp of FP64: FP32 reciprocal square root, a
-// third-order step, and the remainder added back.
+// third-order step, and the remainder added back.  Beyond FP32's range (3e38, a
+// distance of 2e19) the result is no root, but as far away.
 __device__ __forceinline__ double sqrt_f64(double v) {
-    const double y = (double)__builtin_amdgcn_rsqf(fmaxf((float)v, 1e-30f));
+    const double y = (double)__builtin_amdgcn_rsqf(__builtin_amdgcn_fmed3f((float)v, 1e-30f, 3e38f));
     const double g = v * y;
     const double e = fma(-g, y, 1.0);
     const double d = fma(g * e, fma(e, 0.375, 0.5), g);
@@ -207,8 +208,10 @@ __global__ __launch_bounds__(256) void bp_f64(BpArgs a, const double2 *__restric
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const double p = kap * dR[j];
-            const double2 e = cis_rev64((p - rint(p)) + fma(kap, dR[j], -p));
             const bool ok = dR[j] > rmin && dR[j] < rmax;
+            // a pulse outside the gate adds nothing, whatever its range: the phase
+            // factor of one that is no number must not reach the sum either
+            const double2 e = cis_rev64(ok ? (p - rint(p)) + fma(kap, dR[j], -p) : 0.0);
             const double vr = ok ? fma(al[j], sr[j].x - sl[j].x, sl[j].x) : 0.0;
             const double vi = ok ? fma(al[j], sr[j].y - sl[j].y, sl[j].y) : 0.0;
             acc[j].x = fma(vr, e.x, fma(-vi, e.y, acc[j].x));
