@@ -192,7 +192,8 @@ int sarf_backproject(sarf_ctx *ctx, const sarf_bp_desc *desc,
 /* each, one per group but the head group) fit, and an explicit             */
 /* desc->pulse_split that does not fit returns SARF_ERR_INVALID.            */
 /* Every call on one GPU shares that array: calls that overlap on a GPU     */
-/* (other streams, other threads, other contexts) race.  No counterpart in  */
+/* (other streams, other threads, other contexts) race -- but for           */
+/* SARF_BP_F64, which needs no partial images here.  No counterpart in      */
 /* the reference; it is for callers that cannot allocate -- code under HIP  */
 /* graph capture, tight serving loops, harnesses that forbid allocation.    */
 int sarf_backproject_noalloc(sarf_ctx *ctx, const sarf_bp_desc *desc,

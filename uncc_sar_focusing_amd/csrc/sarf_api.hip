@@ -70,6 +70,24 @@ int scratch_get(sarf_ctx *ctx, const char *name, size_t bytes, void **out) {
     return SARF_OK;
 }
 
+static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+}
+
+void *scratch_if_free(sarf_ctx *ctx, const char *name, size_t bytes, hipStream_t s) {
+    {
+        std::lock_guard<std::mutex> lk(ctx->mu);
+        const auto it = ctx->scratch.find(name);
+        if (it != ctx->scratch.end() && it->second.bytes >= bytes) return it->second.ptr;
+    }
+    void *p = nullptr;
+    if (capturing(s) || scratch_get(ctx, name, bytes, &p) == SARF_OK) return p;
+    (void)hipGetLastError();
+    clear_error();
+    return nullptr;
+}
+
 int list_buffer(sarf_ctx *ctx, char tag, const std::vector<unsigned char> &key, size_t bytes,
                 hipStream_t s, const char *who, void **buf, bool *fresh) {
     std::vector<unsigned char> k;
@@ -102,11 +120,6 @@ int list_buffer(sarf_ctx *ctx, char tag, const std::vector<unsigned char> &key, 
     *buf = p;
     *fresh = true;
     return SARF_OK;
-}
-
-static bool capturing(hipStream_t s) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
 }
 
 StreamOrder::StreamOrder(sarf_ctx *c, hipStream_t st) : ctx(c), s(st), active(false) {

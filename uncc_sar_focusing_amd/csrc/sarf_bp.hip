@@ -138,17 +138,18 @@ __device__ __forceinline__ double sqrt_f64(double v) {
 // unrolled.
 constexpr int kF64TX = 32, kF64TY = 16;
 
+// A workgroup per tile and pulse group (img: the partial images of more than one
+// group), or, IN_TURN, one per tile that sums each group by itself and adds the
+// sums in the order of bp_reduce_splits.
+template <bool IN_TURN>
 __global__ __launch_bounds__(256) void bp_f64(BpArgs a, const double2 *__restrict__ prof,
                                               const double *__restrict__ ant,
                                               const double *__restrict__ r0,
                                               const double *__restrict__ f0, double inv_bin,
-                                              double2 *__restrict__ img,
-                                              double2 *__restrict__ part) {
+                                              double2 *__restrict__ img) {
     const int ntiles = a.tiles_x * a.tiles_y;
-    const int split = blockIdx.x / ntiles, t = blockIdx.x - split * ntiles;
+    const int block = blockIdx.x / ntiles, t = blockIdx.x - block * ntiles;
     const int ty = t / a.tiles_x, tx = t - ty * a.tiles_x;
-    int nbeg, nend;
-    split_range(a, split, nbeg, nend);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int x0 = tx * kF64TX + 16 * (wave & 1) + ((lane >> 2) & 3) + 4 * (lane >> 5);
     const int y = ty * kF64TY + 8 * (wave >> 1) + (lane & 3) + 4 * ((lane >> 4) & 1);
@@ -157,49 +158,62 @@ __global__ __launch_bounds__(256) void bp_f64(BpArgs a, const double2 *__restric
     const double px[2] = {a.left + x0 * a.dx, a.left + (x0 + 8) * a.dx};
     const double rmin = -0.5 * a.maxWr, rmax = ((double)(N - 1) / N - 0.5) * a.maxWr;
     const double mid = 0.5 * N;
-    double2 acc[2] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
-    for (int n = nbeg; n < nend; n++) {
-        // wave-uniform: scalar loads
-        const double ax = ant[3 * n], ay = ant[3 * n + 1], az = ant[3 * n + 2], R0 = r0[n];
-        const double kap = f0[n] * (2.0 / kClight);  // revolutions per metre
-        const double2 *__restrict__ row = prof + (size_t)n * N;
-        const double ddy = ay - py;
-        double dR[2];
-        double2 sl[2], sr[2];
-        double al[2];
+    double2 *o = img + (size_t)block * a.split_stride;
+    double2 acc[2] = {}, sum[2] = {};
+    if (IN_TURN && a.accumulate) {
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const double ddx = ax - px[j];
-            dR[j] = sqrt_f64(ddx * ddx + ddy * ddy + az * az) - R0;
-            const double pos = fma(dR[j], inv_bin, mid);
-            // r_0 < dR < r_{N-1} bounds pos to (0, N - 1) up to rounding
-            const int i = (int)fmin(fmax(pos, 0.0), (double)(N - 2));
-            al[j] = pos - (double)i;
-            sl[j] = row[i];
-            sr[j] = row[i + 1];
+        for (int j = 0; j < 2; j++)
+            if (y < a.Ny && x0 + 8 * j < a.Nx) sum[j] = o[(size_t)(x0 + 8 * j) * a.Ny + y];
+    }
+    for (int g = block; g < (IN_TURN ? a.splits : block + 1); g++) {
+        int nbeg, nend;
+        split_range(a, g, nbeg, nend);
+        if (IN_TURN) acc[0] = acc[1] = make_double2(0.0, 0.0);
+        for (int n = nbeg; n < nend; n++) {
+            // wave-uniform: scalar loads
+            const double ax = ant[3 * n], ay = ant[3 * n + 1], az = ant[3 * n + 2], R0 = r0[n];
+            const double kap = f0[n] * (2.0 / kClight);  // revolutions per metre
+            const double2 *__restrict__ row = prof + (size_t)n * N;
+            const double ddy = ay - py;
+            double dR[2];
+            double2 sl[2], sr[2];
+            double al[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const double ddx = ax - px[j];
+                dR[j] = sqrt_f64(ddx * ddx + ddy * ddy + az * az) - R0;
+                const double pos = fma(dR[j], inv_bin, mid);
+                // r_0 < dR < r_{N-1} bounds pos to (0, N - 1) up to rounding
+                const int i = (int)fmin(fmax(pos, 0.0), (double)(N - 2));
+                al[j] = pos - (double)i;
+                sl[j] = row[i];
+                sr[j] = row[i + 1];
+            }
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const double p = kap * dR[j];
+                const bool ok = dR[j] > rmin && dR[j] < rmax;
+                // a pulse outside the gate adds nothing, whatever its range: the phase
+                // factor of one that is no number must not reach the sum either
+                const double2 e = cis_rev64(ok ? (p - rint(p)) + fma(kap, dR[j], -p) : 0.0);
+                const double vr = ok ? fma(al[j], sr[j].x - sl[j].x, sl[j].x) : 0.0;
+                const double vi = ok ? fma(al[j], sr[j].y - sl[j].y, sl[j].y) : 0.0;
+                acc[j].x = fma(vr, e.x, fma(-vi, e.y, acc[j].x));
+                acc[j].y = fma(vr, e.y, fma(vi, e.x, acc[j].y));
+            }
         }
+        if (IN_TURN) {
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const double p = kap * dR[j];
-            const bool ok = dR[j] > rmin && dR[j] < rmax;
-            // a pulse outside the gate adds nothing, whatever its range: the phase
-            // factor of one that is no number must not reach the sum either
-            const double2 e = cis_rev64(ok ? (p - rint(p)) + fma(kap, dR[j], -p) : 0.0);
-            const double vr = ok ? fma(al[j], sr[j].x - sl[j].x, sl[j].x) : 0.0;
-            const double vi = ok ? fma(al[j], sr[j].y - sl[j].y, sl[j].y) : 0.0;
-            acc[j].x = fma(vr, e.x, fma(-vi, e.y, acc[j].x));
-            acc[j].y = fma(vr, e.y, fma(vi, e.x, acc[j].y));
+            for (int j = 0; j < 2; j++) sum[j] = cadd(sum[j], acc[j]);
         }
     }
     if (y >= a.Ny) return;
-    const bool to_part = a.splits > 1;
-    double2 *o = to_part ? part + (size_t)split * a.split_stride : img;
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-        const int x = x0 + 8 * j;
-        if (x >= a.Nx) continue;
-        const size_t idx = (size_t)x * a.Ny + y;
-        o[idx] = a.accumulate && !to_part ? cadd(o[idx], acc[j]) : acc[j];
+        if (x0 + 8 * j >= a.Nx) continue;
+        double2 &v = o[(size_t)(x0 + 8 * j) * a.Ny + y];
+        if (IN_TURN) v = sum[j];
+        else v = a.accumulate ? cadd(v, acc[j]) : acc[j];
     }
 }
 
@@ -608,22 +622,29 @@ int launch_backproject_ext(sarf_ctx *ctx, const sarf_bp_desc *d, const void *pro
         const int want = 8 * (ctx->cu_count > 0 ? ctx->cu_count : 256);
         while (a.splits * ntiles <= want && a.splits < 32 && d->Np / (2 * a.splits) >= 16)
             a.splits *= 2;
+        // Partial images where there is scratch for them.  Without (the allocation-
+        // free entry, a first call under stream capture, a full device) a tile's
+        // workgroup takes the groups in turn, to the same bits
         double2 *part = nullptr;
-        if (a.splits > 1) {
-            const size_t need = sizeof(double2) * (size_t)npix * a.splits;
-            void *buf = ext_part;
-            if (!ext_part) SARF_TRY(scratch_get(ctx, "bp64.partials", need, &buf));
-            else if (need > ext_bytes)
-                return fail(SARF_ERR_INVALID, "backproject: %zu bytes of partial images, more than "
-                            "the %zu available", need, ext_bytes);
-            part = (double2 *)buf;
-            a.split_stride = npix;
+        if (a.splits > 1 && !ext_part)
+            part = (double2 *)scratch_if_free(ctx, "bp64.partials",
+                                              sizeof(double2) * (size_t)npix * a.splits, s);
+        const double2 *p = (const double2 *)prof;
+        const double inv_bin = d->Nfft / d->maxWr;
+        if (a.splits == 1 || part) {
+            BpArgs b = a;
+            if (part) {
+                b.split_stride = npix;
+                b.accumulate = 0;
+            }
+            hipLaunchKernelGGL(bp_f64<false>, dim3((unsigned)(ntiles * a.splits)), dim3(256), 0, s,
+                               b, p, ant, r0, f0, inv_bin, part ? part : (double2 *)img);
+        } else {
+            hipLaunchKernelGGL(bp_f64<true>, dim3((unsigned)ntiles), dim3(256), 0, s, a, p, ant, r0,
+                               f0, inv_bin, (double2 *)img);
         }
-        hipLaunchKernelGGL(bp_f64, dim3((unsigned)(ntiles * a.splits)), dim3(256), 0, s, a,
-                           (const double2 *)prof, ant, r0, f0, d->Nfft / d->maxWr, (double2 *)img,
-                           part);
         SARF_HIP(hipGetLastError());
-        if (a.splits > 1) {
+        if (part) {
             hipLaunchKernelGGL(bp_reduce_splits<double2>, dim3((unsigned)((npix + 255) / 256)),
                                dim3(256), 0, s, part, npix, a.splits, npix, a.accumulate,
                                (double2 *)img);

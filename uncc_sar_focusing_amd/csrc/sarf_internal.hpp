@@ -100,6 +100,9 @@ namespace sarf {
 int use_device(sarf_ctx *ctx);
 // Returns a device buffer of at least `bytes` bytes under `name`.
 int scratch_get(sarf_ctx *ctx, const char *name, size_t bytes, void **out);
+// The same for a caller that can do without: nullptr where the buffer would have
+// to grow while stream s is being captured, or the device is full.
+void *scratch_if_free(sarf_ctx *ctx, const char *name, size_t bytes, hipStream_t s);
 // The device buffer dedicated to one list of a batched entry point: `tag`
 // names the entry point, `key` the caller's list (and parameters that shape
 // the device state).  A list seen before returns its buffer with *fresh =
