@@ -27,3 +27,9 @@ def test_fp64(errors):
     = 1/8, the product by half an ulp of a number below 1, and the steps before
     by less: 4.4e-16 in all, the terms left out 5e-17."""
     assert errors["cis_rev64"] <= 4.4e-16
+
+
+def test_fp32(errors):
+    """The last sum rounds by half an ulp of a number below 1 (3e-8), the squared
+    argument and the product added to it by as much relative to 0.3: 3.6e-8."""
+    assert errors["cis_rev"] <= 6.6e-8

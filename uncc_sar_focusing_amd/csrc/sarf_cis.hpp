@@ -7,6 +7,28 @@
 
 namespace sarf {
 
+// e^{j 2 pi t}, 0 <= t <= 1, within an ulp of FP32 (the sine/cosine unit's
+// absolute error is about four times that): t - q/4 in [-1/8, 1/8] exactly, the
+// Taylor polynomials of sin(2 pi x) and cos(2 pi x) there (the first terms left
+// out are below 3e-9), 2 pi x in two parts, and a quarter turn's exchange and
+// signs.
+__host__ __device__ __forceinline__ float2 cis_rev(float t) {
+    constexpr float kTwoPi = 6.28318548f, kTwoPiRest = -1.74845560e-7f;
+    const float q = rintf(4.f * t);
+    const float x = fmaf(-0.25f, q, t), z = x * x;
+    const float s = fmaf(x, kTwoPi,
+                         x * fmaf(z, fmaf(z, fmaf(z, fmaf(z, 42.058693944897658f, -76.705859753061383f),
+                                                  81.605249276075054f), -41.341702240399755f),
+                                  kTwoPiRest));
+    const float c = fmaf(z, fmaf(z, fmaf(z, fmaf(z, fmaf(z, -26.426256783374398f,
+                                                         60.244641371876663f), -85.456817206693725f),
+                                         64.939394022668291f), -19.739208802178717f), 1.f);
+    const int k = (int)q;
+    const float a = (k & 1) ? s : c, b = (k & 1) ? c : s;  // |cos|, |sin| after the turns
+    // turns 0..4: (c, s), (-s, c), (-c, -s), (s, -c), (c, s)
+    return make_float2(((k + 1) & 2) ? -a : a, (k & 2) ? -b : b);
+}
+
 // e^{j 2 pi t}, |t| <= 1/2 and a little, to an ulp or so of FP64: t - q/4 in
 // [-1/8, 1/8], the Taylor polynomials of sin(2 pi x) to x^15 and cos(2 pi x) to
 // x^16 there (the first terms left out are below 6e-17) and a quarter turn's

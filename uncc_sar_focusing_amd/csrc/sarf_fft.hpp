@@ -5,6 +5,7 @@
 // passes through a padded LDS row).
 #pragma once
 
+#include "sarf_cis.hpp"
 #include "sarf_internal.hpp"
 
 namespace sarf {
@@ -104,6 +105,98 @@ __device__ __forceinline__ void dft(T2 *v) {
     for (int i = 0; i < R; i++) v[i] = t[i];
 }
 
+// cos(2 pi m / 16) less its value rounded to FP64, for m = 1, 2, 3.
+template <int M>
+constexpr double cos16_rest() {
+    constexpr int m = M & 15, f = m > 8 ? 16 - m : m, q = f > 4 ? 8 - f : f;
+    constexpr double t[5] = {0.0, 1.764504708433667706e-17, -4.833646656726456726e-17,
+                             -1.00507726964615876e-17, 0.0};
+    return f > 4 ? -t[q] : t[q];
+}
+
+__device__ __forceinline__ float madd(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double madd(double a, double b, double c) { return fma(a, b, c); }
+
+// rot16<+1, M> with cosine and sine in two parts.  Rounded to FP32, the three
+// constants are all too small, by 1.2e-8 to 2.8e-8, so that every 16-point step
+// shrinks its results: a transform of 2^16, which has four of them, by 5e-8.
+template <int M, typename T2>
+__device__ __forceinline__ T2 rot16_split(T2 d) {
+    constexpr int m = M & 15;
+    if constexpr (m % 4 == 0) {
+        return rot16<+1, m>(d);
+    } else {
+        using Re = decltype(T2{}.x);
+        constexpr double C = Tw16<m>::c(), S = Tw16<m>::s();
+        constexpr Re c = (Re)C, s = (Re)S;
+        constexpr Re cl = (Re)((C - (double)c) + cos16_rest<m>());
+        constexpr Re sl = (Re)((S - (double)s) + cos16_rest<m + 12>());
+        return complex_of(madd(d.x, c, madd(-d.y, s, madd(d.x, cl, -d.y * sl))),
+                          madd(d.x, s, madd(d.y, c, madd(d.x, sl, d.y * cl))));
+    }
+}
+
+template <typename T2>
+__device__ __forceinline__ void idft4(T2 &v0, T2 &v1, T2 &v2, T2 &v3) {
+    const T2 a = cadd(v0, v2), b = csub(v0, v2), c = cadd(v1, v3), d = rot16<+1, 4>(csub(v1, v3));
+    v0 = cadd(a, c);
+    v1 = cadd(b, d);
+    v2 = csub(a, c);
+    v3 = csub(b, d);
+}
+
+// In-place R-point inverse DFT, natural order in and out, with the fewest
+// roundings: radix 4 (one rotation per 16 points where radix 2 has two) and
+// rot16_split.  Transforms of 2^16 samples in FP32: rel-L2 1.23e-7 of this and
+// cis_rev, 1.39e-7 of dft<+1, R>, 1.28e-7 of radix-4 passes with table twiddles.
+template <int R, typename T2>
+__device__ __forceinline__ void idft_split(T2 *v) {
+    static_assert(R == 2 || R == 4 || R == 8 || R == 16, "radix");
+    if constexpr (R == 2) {
+        const T2 a = v[0], b = v[1];
+        v[0] = cadd(a, b);
+        v[1] = csub(a, b);
+    } else if constexpr (R == 4) {
+        idft4(v[0], v[1], v[2], v[3]);
+    } else if constexpr (R == 8) {
+        T2 o[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            o[i] = csub(v[i], v[i + 4]);
+            v[i] = cadd(v[i], v[i + 4]);
+        }
+        o[1] = rot16_split<2>(o[1]);
+        o[2] = rot16_split<4>(o[2]);
+        o[3] = rot16_split<6>(o[3]);
+        idft4(v[0], v[1], v[2], v[3]);
+        idft4(o[0], o[1], o[2], o[3]);
+        v[6] = v[3];
+        v[4] = v[2];
+        v[2] = v[1];
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[2 * i + 1] = o[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) idft4(v[i], v[i + 4], v[i + 8], v[i + 12]);
+        v[5] = rot16_split<1>(v[5]);
+        v[9] = rot16_split<2>(v[9]);
+        v[13] = rot16_split<3>(v[13]);
+        v[6] = rot16_split<2>(v[6]);
+        v[10] = rot16_split<4>(v[10]);
+        v[14] = rot16_split<6>(v[14]);
+        v[7] = rot16_split<3>(v[7]);
+        v[11] = rot16_split<6>(v[11]);
+        v[15] = rot16_split<9>(v[15]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) idft4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+        T2 t[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) t[i] = v[4 * (i & 3) + (i >> 2)];
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[i] = t[i];
+    }
+}
+
 __device__ __forceinline__ int lpad(int i) { return i + (i >> 4); }
 
 // e^{j 2 pi r rev} for r = 1..15 from the sine/cosine unit, which takes
@@ -115,25 +208,6 @@ __device__ __forceinline__ void powers16_rev(float rev, float2 *p) {
         const float a = rev * (float)r;
         p[r] = make_float2(__builtin_amdgcn_cosf(a), __builtin_amdgcn_sinf(a));
     }
-}
-
-// e^{j 2 pi t}, 0 <= t <= 1, within an ulp or so of FP32 (the sine/cosine unit's
-// absolute error is about four times that): t - q/4 in [-1/8, 1/8] exactly, the
-// Taylor polynomials of sin(2 pi x) and cos(2 pi x) there (the first terms left
-// out are below 3e-9), and a quarter turn's exchange and signs.
-__device__ __forceinline__ float2 cis_rev(float t) {
-    const float q = rintf(4.f * t);
-    const float x = fmaf(-0.25f, q, t), z = x * x;
-    const float s = x * fmaf(z, fmaf(z, fmaf(z, fmaf(z, 42.058693944897658f, -76.705859753061383f),
-                                              81.605249276075054f), -41.341702240399755f),
-                             6.2831853071795865f);
-    const float c = fmaf(z, fmaf(z, fmaf(z, fmaf(z, fmaf(z, -26.426256783374398f,
-                                                         60.244641371876663f), -85.456817206693725f),
-                                         64.939394022668291f), -19.739208802178717f), 1.f);
-    const int k = (int)q;
-    const float a = (k & 1) ? s : c, b = (k & 1) ? c : s;  // |cos|, |sin| after the turns
-    // turns 0..4: (c, s), (-s, c), (-c, -s), (s, -c), (c, s)
-    return make_float2(((k + 1) & 2) ? -a : a, (k & 2) ? -b : b);
 }
 
 // w^r for r = 0..15 from w (r = 0 unused); error <= ~4 roundings.

@@ -403,26 +403,25 @@ __global__ __launch_bounds__(pass_threads<T2>()) void rc_pass(PassArgs<T2> p) {
                 const float rev = __builtin_ldexpf((float)k, -(LOG2R + p.log2ns));
 #pragma unroll
                 for (int b = 0; b < RA; b++) {
-                    w[b] = cmul(w[b], fft::cis_rev(__builtin_amdgcn_fractf(
+                    w[b] = cmul(w[b], cis_rev(__builtin_amdgcn_fractf(
                                           rev * (float)(a + R1 * b))));
                 }
             } else {
-                // w^{(a + R1 b) k s}: table entries for a and for b = 1, 2, 4,
-                // 8, the others products of at most four
+                // w^{(a + R1 b) k s}: table entries up to b = 7, one product beyond
                 const long s = (long)k << (p.log2n - LOG2R - p.log2ns);
-                T2 g[16];
-                g[0] = p.twN[a * s];
+                T2 g[RA];
 #pragma unroll
-                for (int b = 1; b < RA; b *= 2) {
-                    const T2 e = p.twN[(long)R1 * b * s & (N - 1)];
+                for (int b = 0; b < RA && b < 8; b++) g[b] = p.twN[(long)(a + R1 * b) * s];
+                if constexpr (RA == 16) {
+                    const T2 e = p.twN[(long)(R1 * 8) * s];
 #pragma unroll
-                    for (int q = 0; q < b; q++) g[b + q] = cmul(g[q], e);
+                    for (int b = 8; b < 16; b++) g[b] = cmul(g[b - 8], e);
                 }
 #pragma unroll
                 for (int b = 0; b < RA; b++) w[b] = cmul(w[b], g[b]);
             }
         }
-        fft::dft<+1, RA>(w);
+        fft::idft_split<RA>(w);
         if (R1 == 1) {
 #pragma unroll
             for (int r = 0; r < RA; r++) store(ci, r, w[r]);
@@ -449,7 +448,7 @@ __global__ __launch_bounds__(pass_threads<T2>()) void rc_pass(PassArgs<T2> p) {
             T2 *w = v + i * R1;
 #pragma unroll
             for (int e = 0; e < R1; e++) w[e] = xch[(e * 16 + q) * CP + c2];
-            fft::dft<+1, R1>(w);
+            fft::idft_split<R1>(w);
         }
 #pragma unroll
         for (int e = 0; e < R1; e++)
@@ -757,6 +756,13 @@ void launch_pass(const PassArgs<T2> &p, int log2r, bool past, long pulses, hipSt
     }
 }
 
+// Passes of a transform of length 2^log2n; in FP64 32 = 8 x 4 instead of one pass
+// of 16 x 2, which rounded once more where few samples are padded to 32.
+template <typename T2>
+int pass_count(int log2n) {
+    return sizeof(T2) == sizeof(double2) && log2n == 5 ? 2 : (log2n + 7) / 8;
+}
+
 // The passes of `pulses` inverse transforms of length 2^log2n (>= 2): p gives
 // the first pass's input and load, the last one's store and output; in between
 // the rows go through x and y in turn (y unused up to two passes, both up to
@@ -764,7 +770,7 @@ void launch_pass(const PassArgs<T2> &p, int log2r, bool past, long pulses, hipSt
 template <typename T2>
 int launch_passes(sarf_ctx *ctx, PassArgs<T2> p, int log2n, long pulses, T2 *x, T2 *y,
                   bool past, hipStream_t s) {
-    const int npass = (log2n + 7) / 8;
+    const int npass = pass_count<T2>(log2n);
     const int load = p.load, store = p.store;
     T2 *const last = p.out;
     p.log2n = log2n;
@@ -799,7 +805,7 @@ template <typename T2>
 int launch_long(sarf_ctx *ctx, const sarf_rc_desc *d, int log2n, const T2 *ph,
                 const float *taper, const double *f0, const double *r0, T2 *prof, hipStream_t s) {
     const size_t row = sizeof(T2) << log2n;
-    const int npass = (log2n + 7) / 8, slab = pulses_per_slab(row, d->Np);
+    const int npass = pass_count<T2>(log2n), slab = pulses_per_slab(row, d->Np);
     const bool past = row * d->Np > kSlabBytes;
     const char *name = sizeof(T2) == sizeof(double2) ? "rc64.tmp" : "rc32.tmp";
     T2 *x = nullptr, *y = nullptr;
@@ -835,7 +841,7 @@ int launch_bluestein_global(sarf_ctx *ctx, const sarf_rc_desc *d, int L, const T
     const T2 *chirp = nullptr, *C = nullptr;
     SARF_TRY(bluestein_tables<T2>(ctx, N, L, &chirp, &C));
     const size_t row = sizeof(T2) << L;
-    const int npass = (L + 7) / 8, slab = pulses_per_slab(row, d->Np);
+    const int npass = pass_count<T2>(L), slab = pulses_per_slab(row, d->Np);
     void *b = nullptr;
     SARF_TRY(scratch_get(ctx, "rcb.rows", row * slab * std::max(2, npass), &b));
     T2 *u = (T2 *)b, *x = u + ((size_t)slab << L), *y = x + ((size_t)slab << L);
