@@ -323,16 +323,16 @@ extern "C" int sarf_bp_entropy_grad(sarf_ctx *ctx, const sarf_bp_desc *d, const 
         case 11: launch_adj_t<32, 4, true>(a, grid, p, ant, r0, f0, im, ent, partial, s); break;
         case 12: launch_adj_t<64, 4, true>(a, grid, p, ant, r0, f0, im, ent, partial, s); break;
         case 13:
-            if (a.narrow) launch_adj_t<64, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, im, ent, partial, s);
+            if (a.five) launch_adj_t<64, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, im, ent, partial, s);
             else launch_adj_t<64, 8, true>(a, grid, p, ant, r0, f0, im, ent, partial, s);
             break;
         case 14: launch_adj_t<32, 8, true>(a, grid, p, ant, r0, f0, im, ent, partial, s); break;
         case 15:
-            if (a.narrow) launch_adj_t<256, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, im, ent, partial, s);
+            if (a.five) launch_adj_t<256, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, im, ent, partial, s);
             else launch_adj_t<256, 8, true>(a, grid, p, ant, r0, f0, im, ent, partial, s);
             break;
         case 16:
-            if (a.narrow) launch_adj_t<128, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, im, ent, partial, s);
+            if (a.five) launch_adj_t<128, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, im, ent, partial, s);
             else launch_adj_t<128, 8, true>(a, grid, p, ant, r0, f0, im, ent, partial, s);
             break;
         default:

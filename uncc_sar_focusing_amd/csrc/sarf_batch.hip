@@ -170,7 +170,7 @@ extern "C" int sarf_bp_batch_entropy(sarf_ctx *ctx, const sarf_bp_desc *d, const
     // persistent: two rounds of the resident workgroups per CU (4, or 5 where
     // the tile's kernel has the smaller windows)
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    const bool five = a.narrow && (tid == 13 || tid == 15 || tid == 16);
+    const bool five = a.five && (tid == 13 || tid == 15 || tid == 16);
     const int grid = (int)std::min<long>(nitems, (five ? 10L : 8L) * cus);
     hipStream_t s = (hipStream_t)stream;
     const float2 *p = (const float2 *)prof;
@@ -183,16 +183,16 @@ extern "C" int sarf_bp_batch_entropy(sarf_ctx *ctx, const sarf_bp_desc *d, const
         case 11: launch_batch_t<32, 4, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
         case 12: launch_batch_t<64, 4, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
         case 13:
-            if (a.narrow) launch_batch_t<64, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            if (a.five) launch_batch_t<64, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
             else launch_batch_t<64, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
             break;
         case 14: launch_batch_t<32, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
         case 15:
-            if (a.narrow) launch_batch_t<256, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            if (a.five) launch_batch_t<256, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
             else launch_batch_t<256, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
             break;
         case 16:
-            if (a.narrow) launch_batch_t<128, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            if (a.five) launch_batch_t<128, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
             else launch_batch_t<128, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
             break;
         default:

@@ -417,6 +417,8 @@ int bp_fill_args(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, BpArgs *out) {
                         "backproject: tile %d spans %.0f range bins (> %d); pixel spacing too "
                         "coarse for the range bin width", tile, wmax, kBpCap);
         a.narrow = wmax <= kBpCapX;
+        // R >= |q|: |q| + |q|^2 / (2 R) <= 3/2 |q|
+        a.five = 1.5 * wmax <= kBpCapX;
         a.tiles_x = (d->Nx + tx - 1) / tx;
         a.tiles_y = (d->Ny + ty - 1) / ty;
     }
@@ -545,7 +547,7 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
     // pulses (tile 16, 760 workgroups) with range compression 48.4 us with the
     // kernel of four waves, which has registers to spare, 49.4 with five; 777 x
     // 603 x 1237 (tile 5, 7904 workgroups) 367 with four, 351 with five
-    const bool five = a.narrow && grid > 4 * (ctx->cu_count > 0 ? ctx->cu_count : 256);
+    const bool five = a.five && grid > 4 * (ctx->cu_count > 0 ? ctx->cu_count : 256);
     const float2 *p = (const float2 *)prof;
     // Tile 15: BpTileU, except for the image a gradient is taken of, whose
     // rounding the adjoint kernel repeats, and where BpTile's larger windows
@@ -570,7 +572,7 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
             break;
         case 14: launch_mixed_t<32, 8, true>(a, grid, p, ant, r0, f0, o, s); break;
         case 15:
-            if (!a.narrow) launch_mixed_t<256, 8, true>(a, grid, p, ant, r0, f0, o, s);
+            if (for_gradient ? !a.five : !a.narrow) launch_mixed_t<256, 8, true>(a, grid, p, ant, r0, f0, o, s);
             else if (for_gradient) launch_mixed_t<256, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
             else launch_mixed_u<256, 8, true>(a, grid, p, ant, r0, f0, o, s);
             break;

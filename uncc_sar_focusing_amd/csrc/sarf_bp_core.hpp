@@ -91,7 +91,10 @@ struct BpArgs {
     double maxWr;
     float invbin;  // Nfft / maxWr (bins per metre)
     double binv;   // the same in FP64
-    int narrow;    // no window of the tile is wider than kBpCapX
+    // Windows against kBpCapX: their bound but for the curvature term |q|^2 / R
+    // (BpTileU, which has a form for wider ones), and with it for any antenna
+    // no nearer than the tile's half diagonal (BpTile, which cuts them there).
+    int narrow, five;
 };
 
 // Pulse range [nbeg, nend) of split s of a tile: even groups, or, with a
