@@ -289,8 +289,8 @@ int sarf_image_entropy(sarf_ctx *ctx, const void *img, /* device complex, npix *
                        double *out, void *stream);
 
 /* ------------------------------------------------------------------------ */
-/* Grid-search objective for many candidate trajectories in one persistent  */
-/* launch.  Candidate c moves each phase centre along a unit direction:     */
+/* Grid-search objective for many candidate trajectories in one launch.     */
+/* Candidate c moves each phase centre along a unit direction:              */
 /*   a_n(c) = a_n + (sum_k coef[c*nbasis + k] * basis[k*Np + n]) * dir_n     */
 /* (e.g. a line-of-sight error a t^2 + b t^3 + c t^4), backprojects all     */
 /* pulses (mixed precision, bp desc as for sarf_backproject) and writes the  */

@@ -262,7 +262,7 @@ class Context:
                       los: tuple[float, float] | None = None,
                       out: torch.Tensor | None = None) -> torch.Tensor:
         """Entropy of the image of every candidate trajectory
-        a_n + (coef[c] . basis[:, n]) * direction[n], one persistent launch.
+        a_n + (coef[c] . basis[:, n]) * direction[n], in one launch.
         `direction` may instead be (nbasis, Np, 3), one field per basis:
         a_n + sum_k coef[c, k] basis[k, n] direction[k, n]."""
         Np, nfft = prof.shape

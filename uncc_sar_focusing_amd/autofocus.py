@@ -1,5 +1,5 @@
 """Autofocus drivers on top of libsarf: batched grid search over trajectory
-candidates (all candidate images of a level in one persistent launch, scored
+candidates (all candidate images of a level in one launch, scored
 by image entropy), multi-resolution refinement with a covariance estimate,
 the trajectory fits that centre the reference's grid, and the
 line-of-sight (LOS) polynomial trajectory model of the batched workload.
@@ -88,7 +88,7 @@ class GridSearchResult:
 def grid_search(ctx, prof: torch.Tensor, ant: torch.Tensor, r0: torch.Tensor, f0: torch.Tensor,
                 grid, maxWr: float, basis: torch.Tensor, direction: torch.Tensor,
                 coefs: np.ndarray, *, los=None, tile: int = 0) -> GridSearchResult:
-    """Evaluate every candidate in `coefs` (ncand, nbasis) in one persistent
+    """Evaluate every candidate in `coefs` (ncand, nbasis) in one
     launch and return the entropy minimiser.  gpu_ms is the device time of the
     launch (HIP events on the stream the work runs on)."""
     dev = prof.device

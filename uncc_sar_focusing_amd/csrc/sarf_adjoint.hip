@@ -82,14 +82,13 @@ __device__ __forceinline__ int scatter_index(int lane) {
 
 constexpr int kWaves = kBpThreads / 64;
 
-template <int TY, int PX, bool XL, int CAP>
+template <int TY, int PX, bool XL>
 __global__ __launch_bounds__(kBpThreads) void bp_entropy_adjoint(
     BpArgs a, const float2 *__restrict__ prof, const double *__restrict__ ant,
     const double *__restrict__ r0, const double *__restrict__ f0, const float2 *__restrict__ img,
     const double *__restrict__ ent, double *__restrict__ partial) {
-    using Tile = BpTile<TY, PX, XL, CAP>;
-    __shared__ typename Tile::Lds L;
-    __shared__ float uz[Tile::CH];
+    __shared__ typename BpTile<TY, PX, XL>::Lds L;
+    __shared__ float uz[BpTile<TY, PX, XL>::CH];
     // blockIdx.x = split * ntiles + tile; each split covers a pulse range
     const int ntiles = a.tiles_x * a.tiles_y;
     const int split = blockIdx.x / ntiles;
@@ -97,7 +96,7 @@ __global__ __launch_bounds__(kBpThreads) void bp_entropy_adjoint(
     const int per_split = (a.Np + a.splits - 1) / a.splits;
     const int nbeg = min(a.Np, split * per_split);
     const int nend = min(a.Np, nbeg + per_split);
-    Tile T;
+    BpTile<TY, PX, XL> T;
     T.init(a, t);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 
@@ -125,7 +124,7 @@ __global__ __launch_bounds__(kBpThreads) void bp_entropy_adjoint(
     const PlainPos pos{ant};
 
     for (int n0 = nbeg; n0 < nend;) {
-        T.stage(a, L, prof, pos, r0, f0, n0, min(Tile::CH, nend - n0));
+        T.stage(a, L, prof, pos, r0, f0, n0, min(BpTile<TY, PX, XL>::CH, nend - n0));
         // uh_z for the chunk (stage() keeps uh_x, uh_y, 1/(2R_c) in pA)
         if (threadIdx.x < L.nc) {
             const int n = n0 + threadIdx.x;
@@ -259,11 +258,11 @@ __global__ __launch_bounds__(64) void adjoint_reduce(const double *__restrict__ 
     }
 }
 
-template <int TY, int PX, bool XL = false, int CAP = kBpCap>
+template <int TY, int PX, bool XL = false>
 void launch_adj_t(const BpArgs &a, int grid, const float2 *prof, const double *ant,
                   const double *r0, const double *f0, const float2 *img, const double *ent,
                   double *partial, hipStream_t s) {
-    hipLaunchKernelGGL((bp_entropy_adjoint<TY, PX, XL, CAP>), dim3(grid), dim3(kBpThreads), 0, s, a, prof,
+    hipLaunchKernelGGL((bp_entropy_adjoint<TY, PX, XL>), dim3(grid), dim3(kBpThreads), 0, s, a, prof,
                        ant, r0, f0, img, ent, partial);
 }
 
@@ -322,19 +321,10 @@ extern "C" int sarf_bp_entropy_grad(sarf_ctx *ctx, const sarf_bp_desc *d, const 
         case 5: launch_adj_t<16, 4>(a, grid, p, ant, r0, f0, im, ent, partial, s); break;
         case 11: launch_adj_t<32, 4, true>(a, grid, p, ant, r0, f0, im, ent, partial, s); break;
         case 12: launch_adj_t<64, 4, true>(a, grid, p, ant, r0, f0, im, ent, partial, s); break;
-        case 13:
-            if (a.five) launch_adj_t<64, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, im, ent, partial, s);
-            else launch_adj_t<64, 8, true>(a, grid, p, ant, r0, f0, im, ent, partial, s);
-            break;
+        case 13: launch_adj_t<64, 8, true>(a, grid, p, ant, r0, f0, im, ent, partial, s); break;
         case 14: launch_adj_t<32, 8, true>(a, grid, p, ant, r0, f0, im, ent, partial, s); break;
-        case 15:
-            if (a.five) launch_adj_t<256, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, im, ent, partial, s);
-            else launch_adj_t<256, 8, true>(a, grid, p, ant, r0, f0, im, ent, partial, s);
-            break;
-        case 16:
-            if (a.five) launch_adj_t<128, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, im, ent, partial, s);
-            else launch_adj_t<128, 8, true>(a, grid, p, ant, r0, f0, im, ent, partial, s);
-            break;
+        case 15: launch_adj_t<256, 8, true>(a, grid, p, ant, r0, f0, im, ent, partial, s); break;
+        case 16: launch_adj_t<128, 8, true>(a, grid, p, ant, r0, f0, im, ent, partial, s); break;
         default:
             return fail(SARF_ERR_UNSUPPORTED, "sarf_bp_entropy_grad: tile %d not compiled", tid);
     }

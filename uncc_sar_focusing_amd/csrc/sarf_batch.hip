@@ -1,4 +1,4 @@
-// sarf_batch.hip -- many candidate images in one persistent launch, scored
+// sarf_batch.hip -- many candidate images in one launch, scored
 // by image entropy without materialising the images.
 //
 // Replaces the grid-search objective of the reference: kernelWrapper
@@ -13,10 +13,12 @@
 // e.g. a line-of-sight polynomial error a t^2 + b t^3 + c t^4, or, with one
 // direction field per basis, a_n(c) = a_n + sum_k coef[c,k] basis[k,n] dir[k,n],
 // which with a_n = 0 and bases 1, i, i^2 along x, y, z is the reference's own
-// absolute trajectory model (:279-291).  A persistent
-// grid walks (tile, candidate) work items, tile-major, so the workgroups
-// resident at one time share a tile and read nearly the same profile windows
-// (L2 reuse).  Each item backprojects all pulses into registers with the
+// absolute trajectory model (:279-291).  One workgroup
+// per (tile, candidate) work item, tile-major, so the workgroups resident at one
+// time share a tile and read nearly the same profile windows (L2 reuse); a
+// persistent grid of two rounds was up to a tenth slower, in whole rounds of
+// work and in registers for its loop (512^2, 128 pulses, 343 candidates 4.94 ms,
+// 4.52 so).  Each item backprojects all pulses into registers with the
 // shared tile engine and reduces S = sum |I|^2 and T = sum |I|^2 ln |I|^2 over
 // the tile into partials[c][tile] (FP64); a second kernel sums the partials
 // in tile order and returns E = ln S - T/S (the entropy of p = |I|^2 / S),
@@ -40,35 +42,33 @@ void bp_batch_entropy(
     BpArgs a, const float2 *__restrict__ prof, const double *__restrict__ ant,
     const double *__restrict__ r0, const double *__restrict__ f0, const double *__restrict__ dir,
     const double *__restrict__ basis, const double *__restrict__ coef, int nbasis, int ncand,
-    int per_basis, double2 *__restrict__ partial) {
+    int per_basis, long first, double2 *__restrict__ partial) {
     using Tile = BpTile<TY, PX, XL, CAP>;
     __shared__ typename Tile::Lds L;
     __shared__ __align__(16) float fx[Tile::kFx];
     __shared__ double2 red[kBpThreads / 64];
     const int ntiles = a.tiles_x * a.tiles_y;
-    const long nitems = (long)ntiles * ncand;
-    for (long item = blockIdx.x; item < nitems; item += gridDim.x) {
-        const int t = (int)(item / ncand);
-        const int c = (int)(item - (long)t * ncand);
-        Tile T;
-        T.init(a, t);
-        LosPolyPos pos{ant, dir, basis, coef + (size_t)c * nbasis, nbasis, a.Np, per_basis};
-        T.run(a, L, fx, prof, pos, r0, f0, 0, a.Np);
-        double s = 0.0, tt = 0.0;
+    const long item = first + blockIdx.x;
+    const int t = (int)(item / ncand);
+    const int c = (int)(item - (long)t * ncand);
+    Tile T;
+    T.init(a, t);
+    LosPolyPos pos{ant, dir, basis, coef + (size_t)c * nbasis, nbasis, a.Np, per_basis};
+    T.run(a, L, fx, prof, pos, r0, f0, 0, a.Np);
+    double s = 0.0, tt = 0.0;
 #pragma unroll
-        for (int j = 0; j < PX; j++) {
-            int x, y;
-            if (T.pixel(j, x, y, a)) {
-                const float m = T.accr[j] * T.accr[j] + T.acci[j] * T.acci[j];
-                if (m > 0.f) {
-                    s += (double)m;
-                    tt += (double)m * (double)__logf(m);
-                }
+    for (int j = 0; j < PX; j++) {
+        int x, y;
+        if (T.pixel(j, x, y, a)) {
+            const float m = T.accr[j] * T.accr[j] + T.acci[j] * T.acci[j];
+            if (m > 0.f) {
+                s += (double)m;
+                tt += (double)m * (double)__logf(m);
             }
         }
-        const double2 r = block_sum2(s, tt, red);
-        if (threadIdx.x == 0) partial[(size_t)c * ntiles + t] = r;
     }
+    const double2 r = block_sum2(s, tt, red);
+    if (threadIdx.x == 0) partial[(size_t)c * ntiles + t] = r;
 }
 
 // E[c] = ln S - T/S from partials[c][0..ntiles), summed in tile order.
@@ -122,13 +122,18 @@ __global__ __launch_bounds__(256) void image_entropy_final(const double2 *__rest
     }
 }
 
+// All items, in launches of at most 2^23 workgroups (a launch holds 2^32 threads).
 template <int TY, int PX, bool XL = false, int CAP = kBpCap>
-void launch_batch_t(const BpArgs &a, int grid, const float2 *prof, const double *ant,
+void launch_batch_t(const BpArgs &a, long nitems, const float2 *prof, const double *ant,
                     const double *r0, const double *f0, const double *dir, const double *basis,
                     const double *coef, int nbasis, int ncand, int per_basis, double2 *partial,
                     hipStream_t s) {
-    hipLaunchKernelGGL((bp_batch_entropy<TY, PX, XL, CAP>), dim3(grid), dim3(kBpThreads), 0, s, a,
-                       prof, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial);
+    constexpr long kMost = 1L << 23;
+    for (long first = 0; first < nitems; first += kMost)
+        hipLaunchKernelGGL((bp_batch_entropy<TY, PX, XL, CAP>),
+                           dim3((unsigned)std::min(kMost, nitems - first)), dim3(kBpThreads), 0, s,
+                           a, prof, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, first,
+                           partial);
 }
 
 }  // namespace
@@ -167,33 +172,29 @@ extern "C" int sarf_bp_batch_entropy(sarf_ctx *ctx, const sarf_bp_desc *d, const
     void *buf = nullptr;
     SARF_TRY(scratch_get(ctx, "batch.partials", sizeof(double2) * (size_t)nitems, &buf));
     double2 *partial = (double2 *)buf;
-    // persistent: two rounds of the resident workgroups per CU (4, or 5 where
-    // the tile's kernel has the smaller windows)
-    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    const bool five = a.five && (tid == 13 || tid == 15 || tid == 16);
-    const int grid = (int)std::min<long>(nitems, (five ? 10L : 8L) * cus);
+    const bool five = bp_five_waves(a, nitems, ctx->cu_count);
     hipStream_t s = (hipStream_t)stream;
     const float2 *p = (const float2 *)prof;
     switch (tid) {
-        case 1: launch_batch_t<32, 4>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
-        case 2: launch_batch_t<64, 4>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
-        case 3: launch_batch_t<64, 8>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
-        case 4: launch_batch_t<32, 8>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
-        case 5: launch_batch_t<16, 4>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
-        case 11: launch_batch_t<32, 4, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
-        case 12: launch_batch_t<64, 4, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
+        case 1: launch_batch_t<32, 4>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
+        case 2: launch_batch_t<64, 4>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
+        case 3: launch_batch_t<64, 8>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
+        case 4: launch_batch_t<32, 8>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
+        case 5: launch_batch_t<16, 4>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
+        case 11: launch_batch_t<32, 4, true>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
+        case 12: launch_batch_t<64, 4, true>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
         case 13:
-            if (a.five) launch_batch_t<64, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
-            else launch_batch_t<64, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            if (five) launch_batch_t<64, 8, true, kBpCapX>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            else launch_batch_t<64, 8, true>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
             break;
-        case 14: launch_batch_t<32, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
+        case 14: launch_batch_t<32, 8, true>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s); break;
         case 15:
-            if (a.five) launch_batch_t<256, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
-            else launch_batch_t<256, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            if (five) launch_batch_t<256, 8, true, kBpCapX>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            else launch_batch_t<256, 8, true>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
             break;
         case 16:
-            if (a.five) launch_batch_t<128, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
-            else launch_batch_t<128, 8, true>(a, grid, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            if (five) launch_batch_t<128, 8, true, kBpCapX>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
+            else launch_batch_t<128, 8, true>(a, nitems, p, ant, r0, f0, dir, basis, coef, nbasis, ncand, per_basis, partial, s);
             break;
         default:
             return fail(SARF_ERR_UNSUPPORTED, "sarf_bp_batch_entropy: tile %d not compiled for batches", tid);

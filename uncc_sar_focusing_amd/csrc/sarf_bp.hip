@@ -543,11 +543,7 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
         a.split_stride = npix;
     }
     const int grid = ntiles * splits;
-    // five waves per SIMD where there are workgroups for the fifth: 605 x 597, 94
-    // pulses (tile 16, 760 workgroups) with range compression 48.4 us with the
-    // kernel of four waves, which has registers to spare, 49.4 with five; 777 x
-    // 603 x 1237 (tile 5, 7904 workgroups) 367 with four, 351 with five
-    const bool five = a.five && grid > 4 * (ctx->cu_count > 0 ? ctx->cu_count : 256);
+    const bool five = bp_five_waves(a, grid, ctx->cu_count);
     const float2 *p = (const float2 *)prof;
     // Tile 15: BpTileU, except for the image a gradient is taken of, whose
     // rounding the adjoint kernel repeats, and where BpTile's larger windows
@@ -572,8 +568,8 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
             break;
         case 14: launch_mixed_t<32, 8, true>(a, grid, p, ant, r0, f0, o, s); break;
         case 15:
-            if (for_gradient ? !a.five : !a.narrow) launch_mixed_t<256, 8, true>(a, grid, p, ant, r0, f0, o, s);
-            else if (for_gradient) launch_mixed_t<256, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
+            if (for_gradient && five) launch_mixed_t<256, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
+            else if (for_gradient || !a.narrow) launch_mixed_t<256, 8, true>(a, grid, p, ant, r0, f0, o, s);
             else launch_mixed_u<256, 8, true>(a, grid, p, ant, r0, f0, o, s);
             break;
         case 16:

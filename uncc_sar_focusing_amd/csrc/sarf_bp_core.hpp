@@ -66,9 +66,10 @@ static_assert(kBpChunk <= 64 && kBpCap % kBpThreads == 0, "staging layout");
 // 8 pixels per lane, except lanes-along-x tiles whose column terms take the
 // LDS past 40 KiB (3 workgroups per CU); the 16-pixel tiles need more
 // registers than that.  Tiles 5, 13, 15 and 16 with the smaller windows: 5 (2048^2
-// at 0.05 m, 4096 pulses, tile 16 6.98 -> 6.74 ms, tile 13 7.23 -> 6.94; 1331
-// candidates at 512^2, 1024 pulses, tile 15 154.0 -> 150.2 ms, 153.7 with 4; 777 x
-// 603, 1237 pulses, tile 5 with range compression 367 -> 352 us).
+// at 0.05 m, 4096 pulses, tile 16 6.98 -> 6.74 ms, tile 13 7.23 -> 6.94; 343
+// candidates at 512^2, 128 pulses, tile 15 4.52 -> 4.48 ms; 777 x 603, 1237 pulses,
+// tile 5 with range compression 367 -> 352 us); which launches take them is
+// bp_five_waves.
 template <int TY, int PX, bool XL, int CAP = kBpCap>
 constexpr int bp_waves_per_eu() {
     return CAP < kBpCap ? 5 : PX > 8 ? 1 : (XL && (kBpThreads / TY) * PX > 32) ? 3 : 4;
@@ -96,6 +97,19 @@ struct BpArgs {
     // no nearer than the tile's half diagonal (BpTile, which cuts them there).
     int narrow, five;
 };
+
+// Whether a launch of `groups` workgroups of tile 5, 13, 15 or 16 takes BpTile's
+// kernel for five waves per SIMD.  That has fewer registers (it spills) and a
+// smaller window buffer, so it pays only where the fifth wave has work: more
+// than eight workgroups per CU.  Measured with four waves and five (us, 256 CUs):
+// images of 1536 workgroups 137.6 / 140.2 (211 x 186, 1611 pulses, tile 5), 1728
+// 61.2 / 62.5 (537 x 362, 263, tile 13), 2912 58.8 / 56.9 (415 x 410, 307, tile 5),
+// 4248 83.7 / 79.6 (1095 x 931, 90); candidate batches of 750 workgroups 110.0 /
+// 115.0, 1600 212 / 215, 2048 239 / 241, 2457 307 / 305, 6250 718 / 703, 43904
+// 4518 / 4476 (128 pulses).
+inline bool bp_five_waves(const BpArgs &a, long groups, int cus) {
+    return a.five && groups > 8L * (cus > 0 ? cus : 256);
+}
 
 // Pulse range [nbeg, nend) of split s of a tile: even groups, or, with a
 // tail, one head group of the first Np - tail pulses and the tail pulses in
