@@ -1,5 +1,6 @@
-"""Rounding of the global-memory range-compression passes against long double: no
-more than that of radix-4 passes with every twiddle from a table."""
+"""Rounding of range compression against long double: through global memory no more
+than that of radix-4 passes with every twiddle from a table, at lengths that are no
+power of two no more than that of the longer convolution."""
 import numpy as np
 import pytest
 import torch
@@ -29,3 +30,17 @@ def test_fp32(ctx, nfft, tol):
                                            (50, 410, 4096, 3.2e-16)])
 def test_fp64(ctx, Np, K, nfft, tol):
     assert _error(ctx, Np, K, nfft, np.complex128) <= tol
+
+
+# Lengths that are no power of two.  The bounds are the errors of plain transforms of the
+# length for 2 N - 1, whatever K, in the register-resident kernel and in radix-4 passes.
+@pytest.mark.parametrize("N,K,tol", [(37, 28, 1.30e-7), (65, 64, 1.62e-7), (300, 213, 1.79e-7),
+                                     (1025, 1024, 2.35e-7), (3000, 731, 2.77e-7),
+                                     (4097, 4096, 4.2e-7), (20011, 3000, 1.73e-7)])
+def test_fp32_other_lengths(ctx, N, K, tol):
+    assert _error(ctx, 400 if N < 2000 else 20, K, N, np.complex64) <= tol
+
+
+@pytest.mark.parametrize("N,K,tol", [(3000, 700, 6.8e-16)])
+def test_fp64_other_lengths(ctx, N, K, tol):
+    assert _error(ctx, 20, K, N, np.complex128) <= tol

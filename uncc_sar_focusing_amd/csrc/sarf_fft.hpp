@@ -270,8 +270,9 @@ struct Shape {
 // Starts with a barrier, so the caller may have just read L; every thread
 // of the workgroup must call it.  The forward transform is conj(ifft(conj)).
 // With active = false a thread only takes part in the barriers (for a
-// workgroup wider than the row's T lanes); its v is left unchanged.
-template <int LOG2N>
+// workgroup wider than the row's T lanes); its v is left unchanged.  SPLIT: by
+// idft_split.
+template <int LOG2N, bool SPLIT = false>
 __device__ __forceinline__ void ifft_regs(float2 (&v)[16], float2 *L, int j,
                                           const float2 *__restrict__ tw, bool active = true) {
     using S = Shape<LOG2N>;
@@ -281,7 +282,8 @@ __device__ __forceinline__ void ifft_regs(float2 (&v)[16], float2 *L, int j,
 #pragma unroll
         for (int b = 0; b < NB0; b++) {
             const int jb = j + b * T;
-            dft<+1, R0>(v + b * R0);
+            if constexpr (SPLIT) idft_split<R0>(v + b * R0);
+            else dft<+1, R0>(v + b * R0);
 #pragma unroll
             for (int r = 0; r < R0; r++) L[lpad(jb * R0 + r)] = v[b * R0 + r];
         }
@@ -301,7 +303,8 @@ __device__ __forceinline__ void ifft_regs(float2 (&v)[16], float2 *L, int j,
 #pragma unroll
                 for (int r = 1; r < 16; r++) v[r] = cmul(v[r], p[r]);
             }
-            dft<+1, 16>(v);
+            if constexpr (SPLIT) idft_split<16>(v);
+            else dft<+1, 16>(v);
         }
         if (!last) {
             __syncthreads();  // every lane has read before anyone overwrites

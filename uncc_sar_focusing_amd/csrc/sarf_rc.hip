@@ -42,6 +42,14 @@ using fft::pass_twiddles;
 // Bluestein kernel (M <= 16384); longer ones (and FP64) go through the
 // global-memory passes, up to 2^20 (M = 2^21).
 constexpr int kBluesteinMaxN = 8192;
+// Shortest one whose M follows N + K - 1 instead of 2 N - 1.  A shorter convolution
+// spreads its rounding over fewer outputs, up to half of which were discarded: as
+// much as sqrt(2) more of it in the profiles.  Transforms by idft_split make up
+// for that from here on (rel-L2 at N = 65, K = 64 1.52e-7, M = 256 without either
+// 1.62e-7; 4097, 4096 2.3e-7 and 4.2e-7; 33, 32 1.33e-7 and 1.24e-7); the passes
+// through global memory, which had them already, keep 2 N - 1 (20011, 3000:
+// 1.72e-7, with the shorter one 1.92e-7).
+constexpr int kBluesteinShortN = 65;
 constexpr int kBluesteinGlobalMaxN = 1 << 20;
 
 constexpr int rc_threads(int log2n) {
@@ -462,17 +470,18 @@ __global__ __launch_bounds__(pass_threads<T2>()) void rc_pass(PassArgs<T2> p) {
 // N_fft = K, charlotte_sar_api.hpp:173): Bluestein's identity
 // k m = (k^2 + m^2 - (m - k)^2) / 2 turns the length-N inverse DFT into a
 // circular convolution of length M = 2^ceil(log2(N + K - 1)) (the K samples
-// meet chirp offsets -(K - 1) .. N - 1):
+// meet chirp offsets -(K - 1) .. N - 1; below kBluesteinShortN with K = N):
 //   X_m = c_m sum_k (x_k c_k) conj(c_{m-k}),   c_k = e^{+j pi k^2 / N},
 // formed per pulse by two register-resident radix-16 transforms of length M
 // (sarf_fft.hpp): the forward transform of a_k = x_k c_k as conj(ifft(conj)),
-// the product with C = FFT_M(conj(c)) (a per-N table, circularly extended),
+// the product with C = FFT_M(conj(c)) (a table per N and M, circularly extended),
 // and the inverse transform.  c_k comes from the exact k^2 mod 2N in FP64.
 // Zero padding (k >= K) is never loaded; fftshift = cshift((N+1)/2) is an
 // index remap on the store (odd N included), with 1/N and the ramp.  One row
 // of M/16 lanes per pulse, rows packed to >= 256 lanes per workgroup.
+// SPLIT: transforms by idft_split.
 // ---------------------------------------------------------------------------
-template <int LOG2M>
+template <int LOG2M, bool SPLIT>
 __global__ __launch_bounds__(fft::group_threads(LOG2M))
 __attribute__((amdgpu_waves_per_eu(LOG2M <= 13 ? 4 : 1))) void rc_bluestein(
     const float2 *__restrict__ ph, int K, int N, int Np, int flags,
@@ -515,12 +524,12 @@ __attribute__((amdgpu_waves_per_eu(LOG2M <= 13 ? 4 : 1))) void rc_bluestein(
             }
             v[b * S::R0 + r] = make_float2(a.x, -a.y);
         }
-    fft::ifft_regs<LOG2M>(v, Lr, j, twM);  // v[r] = conj(A_k), k = j + r*T
+    fft::ifft_regs<LOG2M, SPLIT>(v, Lr, j, twM);  // v[r] = conj(A_k), k = j + r*T
     float2 u[16];
 #pragma unroll
     for (int r = 0; r < 16; r++) u[r] = cmul(make_float2(v[r].x, -v[r].y), C[j + r * T]);
     fft::to_input_order<LOG2M>(u, v);
-    fft::ifft_regs<LOG2M>(v, Lr, j, twM);  // v[r] = M (a * conj c)_{j + r*T}
+    fft::ifft_regs<LOG2M, SPLIT>(v, Lr, j, twM);  // v[r] = M (a * conj c)_{j + r*T}
     if (!active) return;
     const float fr = ramp[lp].x, fi = ramp[lp].y;
     const int half = (N + 1) / 2;
@@ -716,13 +725,18 @@ int bluestein_tables(sarf_ctx *ctx, int N, int L, const T2 **chirp, const T2 **C
 }
 
 template <int LOG2M>
-void launch_bluestein_t(const sarf_rc_desc *d, const float2 *ph, const float *taper,
+void launch_bluestein_t(const sarf_rc_desc *d, bool split, const float2 *ph, const float *taper,
                         const double *f0, const double *r0, const float2 *chirp, const float2 *C,
                         const float2 *tw, float2 *prof, hipStream_t s) {
     constexpr int P = fft::rows_per_group(LOG2M);
-    hipLaunchKernelGGL(rc_bluestein<LOG2M>, dim3((d->Np + P - 1) / P),
-                       dim3(fft::group_threads(LOG2M)), 0, s, ph, d->K, d->Nfft, d->Np, d->flags,
-                       taper, f0, r0, chirp, C, tw, prof);
+    const auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((d->Np + P - 1) / P), dim3(fft::group_threads(LOG2M)), 0, s,
+                           ph, d->K, d->Nfft, d->Np, d->flags, taper, f0, r0, chirp, C, tw, prof);
+    };
+    if constexpr (LOG2M < 14) {  // 2^14 is nobody's shorter length
+        if (split) return run(rc_bluestein<LOG2M, true>);
+    }
+    run(rc_bluestein<LOG2M, false>);
 }
 
 template <typename T2>
@@ -891,24 +905,26 @@ int launch_range_compress(sarf_ctx *ctx, const sarf_rc_desc *d, const void *ph,
     const bool f64 = (d->flags & SARF_RC_F64) != 0;
     if (log2n < 0 && !f64 && d->Nfft <= kBluesteinMaxN) {
         // not a power of two: Bluestein through two register-resident
-        // transforms of length M
-        const int L = bluestein_log2(d->Nfft, d->K, 5);
+        // transforms of length M, by idft_split if that is the shorter one
+        const int full = bluestein_log2(d->Nfft, d->Nfft, 5);
+        const int L = d->Nfft < kBluesteinShortN ? full : bluestein_log2(d->Nfft, d->K, 5);
+        const bool split = L < full;
         const float2 *chirp = nullptr, *C = nullptr, *tw = nullptr;
         SARF_TRY(bluestein_tables<float2>(ctx, d->Nfft, L, &chirp, &C));
         SARF_TRY(twiddles_f32(ctx, L, &tw));
         const float2 *x = (const float2 *)ph;
         float2 *y = (float2 *)prof;
         switch (L) {
-            case 5: launch_bluestein_t<5>(d, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 6: launch_bluestein_t<6>(d, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 7: launch_bluestein_t<7>(d, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 8: launch_bluestein_t<8>(d, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 9: launch_bluestein_t<9>(d, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 10: launch_bluestein_t<10>(d, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 11: launch_bluestein_t<11>(d, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 12: launch_bluestein_t<12>(d, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 13: launch_bluestein_t<13>(d, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 14: launch_bluestein_t<14>(d, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 5: launch_bluestein_t<5>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 6: launch_bluestein_t<6>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 7: launch_bluestein_t<7>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 8: launch_bluestein_t<8>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 9: launch_bluestein_t<9>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 10: launch_bluestein_t<10>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 11: launch_bluestein_t<11>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 12: launch_bluestein_t<12>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 13: launch_bluestein_t<13>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 14: launch_bluestein_t<14>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
             default: return fail(SARF_ERR_UNSUPPORTED, "range_compress: Nfft=%d", d->Nfft);
         }
         SARF_HIP(hipGetLastError());
@@ -920,7 +936,7 @@ int launch_range_compress(sarf_ctx *ctx, const sarf_rc_desc *d, const void *ph,
         if (d->Nfft > kBluesteinGlobalMaxN)
             return fail(SARF_ERR_UNSUPPORTED, "range_compress: Nfft=%d (lengths that are not a "
                         "power of two go up to %d)", d->Nfft, kBluesteinGlobalMaxN);
-        const int L = bluestein_log2(d->Nfft, d->K, 1);
+        const int L = bluestein_log2(d->Nfft, d->Nfft, 1);
         if (f64)
             return launch_bluestein_global<double2>(ctx, d, L, (const double2 *)ph, taper, f0, r0,
                                                     (double2 *)prof, s);
