@@ -479,11 +479,12 @@ __global__ __launch_bounds__(pass_threads<T2>()) void rc_pass(PassArgs<T2> p) {
 // Zero padding (k >= K) is never loaded; fftshift = cshift((N+1)/2) is an
 // index remap on the store (odd N included), with 1/N and the ramp.  One row
 // of M/16 lanes per pulse, rows packed to >= 256 lanes per workgroup.
-// SPLIT: transforms by idft_split.
+// SPLIT: transforms by idft_split.  FOUR (M = 2^12, 2^13): four waves per SIMD, which
+// takes spills that the form of three waves does not need.
 // ---------------------------------------------------------------------------
-template <int LOG2M, bool SPLIT>
+template <int LOG2M, bool SPLIT, bool FOUR>
 __global__ __launch_bounds__(fft::group_threads(LOG2M))
-__attribute__((amdgpu_waves_per_eu(LOG2M <= 13 ? 4 : 1))) void rc_bluestein(
+__attribute__((amdgpu_waves_per_eu(LOG2M <= 11 || FOUR ? 4 : 1))) void rc_bluestein(
     const float2 *__restrict__ ph, int K, int N, int Np, int flags,
     const float *__restrict__ taper, const double *__restrict__ f0,
     const double *__restrict__ r0, const float2 *__restrict__ chirp,
@@ -724,19 +725,31 @@ int bluestein_tables(sarf_ctx *ctx, int N, int L, const T2 **chirp, const T2 **C
     return SARF_OK;
 }
 
+// At 2^12 and 2^13 the kernel of four waves where there are pulses for it (a
+// workgroup is one or two waves per SIMD): 1314 samples and bins, 500 pulses 15.0
+// us with the other, 15.8 with this, 800 pulses 22.5 and 20.7; 2957 bins of 1147
+// samples, 195 pulses 16.4 and 19.4, 300 pulses 26.7 and 24.5, 2500 pulses 119 and 93.
 template <int LOG2M>
-void launch_bluestein_t(const sarf_rc_desc *d, bool split, const float2 *ph, const float *taper,
-                        const double *f0, const double *r0, const float2 *chirp, const float2 *C,
-                        const float2 *tw, float2 *prof, hipStream_t s) {
+void launch_bluestein_t(const sarf_rc_desc *d, bool split, int cus, const float2 *ph,
+                        const float *taper, const double *f0, const double *r0,
+                        const float2 *chirp, const float2 *C, const float2 *tw, float2 *prof,
+                        hipStream_t s) {
     constexpr int P = fft::rows_per_group(LOG2M);
+    constexpr bool kBoth = LOG2M == 12 || LOG2M == 13;
+    const bool four = kBoth && d->Np > (LOG2M == 12 ? 3 : 1) * (cus > 0 ? cus : 256);
     const auto run = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((d->Np + P - 1) / P), dim3(fft::group_threads(LOG2M)), 0, s,
                            ph, d->K, d->Nfft, d->Np, d->flags, taper, f0, r0, chirp, C, tw, prof);
     };
     if constexpr (LOG2M < 14) {  // 2^14 is nobody's shorter length
-        if (split) return run(rc_bluestein<LOG2M, true>);
+        if (split) {
+            if (four) run(rc_bluestein<LOG2M, true, kBoth>);
+            else run(rc_bluestein<LOG2M, true, false>);
+            return;
+        }
     }
-    run(rc_bluestein<LOG2M, false>);
+    if (four) run(rc_bluestein<LOG2M, false, kBoth>);
+    else run(rc_bluestein<LOG2M, false, false>);
 }
 
 template <typename T2>
@@ -909,22 +922,23 @@ int launch_range_compress(sarf_ctx *ctx, const sarf_rc_desc *d, const void *ph,
         const int full = bluestein_log2(d->Nfft, d->Nfft, 5);
         const int L = d->Nfft < kBluesteinShortN ? full : bluestein_log2(d->Nfft, d->K, 5);
         const bool split = L < full;
+        const int cus = ctx->cu_count;
         const float2 *chirp = nullptr, *C = nullptr, *tw = nullptr;
         SARF_TRY(bluestein_tables<float2>(ctx, d->Nfft, L, &chirp, &C));
         SARF_TRY(twiddles_f32(ctx, L, &tw));
         const float2 *x = (const float2 *)ph;
         float2 *y = (float2 *)prof;
         switch (L) {
-            case 5: launch_bluestein_t<5>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 6: launch_bluestein_t<6>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 7: launch_bluestein_t<7>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 8: launch_bluestein_t<8>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 9: launch_bluestein_t<9>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 10: launch_bluestein_t<10>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 11: launch_bluestein_t<11>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 12: launch_bluestein_t<12>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 13: launch_bluestein_t<13>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
-            case 14: launch_bluestein_t<14>(d, split, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 5: launch_bluestein_t<5>(d, split, cus, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 6: launch_bluestein_t<6>(d, split, cus, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 7: launch_bluestein_t<7>(d, split, cus, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 8: launch_bluestein_t<8>(d, split, cus, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 9: launch_bluestein_t<9>(d, split, cus, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 10: launch_bluestein_t<10>(d, split, cus, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 11: launch_bluestein_t<11>(d, split, cus, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 12: launch_bluestein_t<12>(d, split, cus, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 13: launch_bluestein_t<13>(d, split, cus, x, taper, f0, r0, chirp, C, tw, y, s); break;
+            case 14: launch_bluestein_t<14>(d, split, cus, x, taper, f0, r0, chirp, C, tw, y, s); break;
             default: return fail(SARF_ERR_UNSUPPORTED, "range_compress: Nfft=%d", d->Nfft);
         }
         SARF_HIP(hipGetLastError());
