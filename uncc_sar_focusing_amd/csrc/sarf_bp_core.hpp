@@ -368,9 +368,9 @@ struct BpTile {
                                         (float)(g1 * up * mp), 0.f);
             }
             // Fast path: the window lies inside the profile (no swath gate) and
-            // |psi| <= 0.5 + kap * ext stays inside v_sin/v_cos's input range
+            // |psi| <= 0.5 + |kap| * ext stays inside v_sin/v_cos's input range
             // (|x| <= 256 revolutions), so the phase needs no reduction.
-            interior = (st >= 0 && st + W <= a.Nfft && kap * ext <= 250.0) ? 1 : 0;
+            interior = (st >= 0 && st + W <= a.Nfft && fabs(kap) * ext <= 250.0) ? 1 : 0;
         }
         if (tid < 64) {
             // Windows are packed back to back: offsets are the exclusive
@@ -690,7 +690,7 @@ struct BpTileU {
                                 (float)(a.binv / kap), (float)(posg - st - kBinShift), 0.f);
                 L.pA[tid] = make_float4((float)ah, (float)bh, (float)g0, (float)g1);
                 L.kap[tid] = (float)kap;
-                const bool inside = st >= 0.0 && st + wd <= a.Nfft && kap * ext <= 250.0;
+                const bool inside = st >= 0.0 && st + wd <= a.Nfft && fabs(kap) * ext <= 250.0;
                 mode = inside ? kPulseFast : kPulseGated;
                 // half extent along the pixel axis; the cubic term there in
                 // revolutions, and a carrier so low that the phase cannot
