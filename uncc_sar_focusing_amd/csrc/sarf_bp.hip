@@ -468,11 +468,16 @@ std::array<uint64_t, 8> tune_key(const sarf_bp_desc *d) { return tune_key(tune_g
 //   (a tail of 1/4, 1/6, 1/12 or 1/16 of the pulses measured 7.27-7.58 ms);
 // * even groups otherwise (few tiles: the groups are what fills the GPU),
 //   doubling until there are 16 workgroups per CU with at least 16 pulses
-//   per group.  Every group costs a partial image written and read again: 1024^2
-//   x 896 pulses (512 tiles) 361 us with 8 groups, 416 with 32; 1400 x 1000 x 600
-//   (693 tiles) 390 with 8, 503 with 32; 777 x 603 x 1237 (494 tiles) 304 with
-//   16, 323 with 32; 768^2 x 1000 (288) 232 with 16, 254 with 32; 512^2 x 1024
-//   (128) 118 with 16, 123 with 32; 256^2 x 512 (32) 34 with 16 to 32.
+//   per group, and on to 64 per CU while groups keep at least 112 pulses.  Every
+//   group costs a partial image written and read again: 1024^2 x 896 pulses (512
+//   tiles) 361 us with 8 groups, 416 with 32; 1400 x 1000 x 600 (693 tiles) 390
+//   with 8, 503 with 32; 777 x 603 x 1237 (494 tiles) 304 with 16, 323 with 32.
+//   With long groups that is little beside what the last, partly filled round
+//   of workgroups takes: 1028 x 1349 x 2361 (1419 tiles) 1825 us with 16, 2012
+//   with 4; 1632 x 1428 x 2511 (1170) 2890 with 16, 3044 with 4; 1861 x 1124 x
+//   3470 (1080) 3380 with 16, 3490 with 4 (range compression included).  Over 60
+//   images of 79 to 1847 pixels a side the least pulses for that measured the
+//   same from 64 to 128.
 
 bool split_head_tail(const sarf_ctx *ctx, int tile, int ntiles, int Np) {
     const long resident = (long)(ctx->cu_count > 0 ? ctx->cu_count : 256) * tile_waves_per_eu(tile);
@@ -488,8 +493,10 @@ int default_splits(const sarf_ctx *ctx, int tile, int ntiles, int Np, bool for_g
     if (split_head_tail(ctx, tile, ntiles, Np)) return 3;
     int splits = 1;
     const long cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    const long want = (for_gradient ? 64L : 16L) * cus;
-    while (splits < 32 && (long)ntiles * splits < want && Np / (2 * splits) >= 16) splits *= 2;
+    const auto least = [&](long groups) { return for_gradient || groups < 16 * cus ? 16 : 112; };
+    while (splits < 32 && (long)ntiles * splits < 64 * cus &&
+           Np / (2 * splits) >= least((long)ntiles * splits))
+        splits *= 2;
     while (!for_gradient && splits < 32 && (long)ntiles * splits < cus && Np / (2 * splits) >= 4)
         splits *= 2;
     return splits;
