@@ -49,8 +49,9 @@ extern "C" {
 
 /* backprojection flags */
 #define SARF_BP_ACCUMULATE 1 /* add into img instead of overwriting it */
-#define SARF_BP_FOR_GRADIENT 4 /* sarf_backproject: round as sarf_bp_entropy_grad's recomputation
-                                  and sarf_bp_batch_entropy do (a little slower and coarser) */
+#define SARF_BP_FOR_GRADIENT 4 /* sarf_backproject: range expansion and rounding of
+                                  sarf_bp_entropy_grad's recomputation and of
+                                  sarf_bp_batch_entropy (a little slower and coarser) */
 #define SARF_BATCH_DIR_PER_BASIS 2 /* sarf_bp_batch_entropy: dir holds one field per basis */
 #define SARF_SCENES_TILE_MIXED 100 /* sarf_bp_scenes: a tile per scene (see there) */
 
@@ -239,7 +240,9 @@ int sarf_matched_filter(sarf_ctx *ctx, const sarf_mf_desc *desc,
 /* spacing, maxWr, LOS hint): later sarf_backproject calls with tile = 0 and */
 /* pulse_split = 0 use it.  On return img holds the backprojection made     */
 /* with the chosen pair.  desc->flags must not hold SARF_BP_ACCUMULATE;     */
-/* desc->tile and desc->pulse_split are ignored.  No reference counterpart: */
+/* desc->tile, desc->pulse_split and SARF_BP_FOR_GRADIENT are ignored.  A    */
+/* call with SARF_BP_FOR_GRADIENT uses the remembered tile only: its pulses */
+/* are grouped by the default rule.  No reference counterpart:              */
 /* the reference launches one fixed block shape (src/gpuBackProjection/     */
 /* cuda_sar_focusing/cuda_sar_focusing.hpp:632-634).                        */
 /* ------------------------------------------------------------------------ */

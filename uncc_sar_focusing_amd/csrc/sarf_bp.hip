@@ -487,8 +487,8 @@ bool split_head_tail(const sarf_ctx *ctx, int tile, int ntiles, int Np) {
 // Where that leaves CUs without a workgroup (the smallest images), on down to
 // 4 pulses per group: a lone workgroup's time is its chain of LDS and memory
 // latencies per pulse (128^2 x 117 pulses, 8 tiles: 4 groups 27.8 us, 8 groups
-// 20.5, 16 groups 15.8, 32 groups 16.1).  The image a gradient is taken of is
-// rounded as it always was: up to 64 workgroups per CU, 16 pulses or more.
+// 20.5, 16 groups 15.8, 32 groups 16.1).  The image a gradient is taken of has one
+// rule whatever its size: up to 64 workgroups per CU, 16 pulses or more.
 int default_splits(const sarf_ctx *ctx, int tile, int ntiles, int Np, bool for_gradient) {
     if (split_head_tail(ctx, tile, ntiles, Np)) return 3;
     int splits = 1;
@@ -664,7 +664,9 @@ int launch_backproject_ext(sarf_ctx *ctx, const sarf_bp_desc *d, const void *pro
         auto it = ctx->tuned.find(tune_key(d));
         if (it != ctx->tuned.end()) {
             tile = it->second.tile;
-            splits = it->second.pulse_split;
+            // the groups of an image a gradient is taken of follow the rule,
+            // whatever was measured for other images
+            if (!(d->flags & SARF_BP_FOR_GRADIENT)) splits = it->second.pulse_split;
         }
     }
     if (tile == 0) {
@@ -737,6 +739,7 @@ extern "C" int sarf_autotune(sarf_ctx *ctx, const sarf_bp_desc *d, const void *p
     SARF_TRY(bp_fill_args(ctx, d, 0, &chk));  // validates sizes and geometry
     hipStream_t s = (hipStream_t)stream;
     sarf_bp_desc dd = *d;
+    dd.flags &= ~SARF_BP_FOR_GRADIENT;  // shapes are measured for and used by other images
     dd.tile = 0;
     dd.pulse_split = 0;
     EventPair ev;
