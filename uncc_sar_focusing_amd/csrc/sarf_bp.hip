@@ -70,16 +70,15 @@ void bp_mixed(BpArgs a, const float2 *__restrict__ prof,
 }
 
 // The same over BpTileU.
-template <int TL, int PX, bool XL>
 __global__ __launch_bounds__(kBpThreads) __attribute__((amdgpu_waves_per_eu(kBpWavesU)))
 void bp_mixed_u(BpArgs a, const float2 *__restrict__ prof, const double *__restrict__ ant,
                 const double *__restrict__ r0, const double *__restrict__ f0,
                 float2 *__restrict__ img) {
-    __shared__ typename BpTileU<TL, PX, XL>::Lds L;
+    __shared__ BpLdsU L;
     int nbeg, nend, accumulate;
     float2 *out = img;
     const int t = split_block(a, out, accumulate, nbeg, nend);
-    BpTileU<TL, PX, XL> T;
+    BpTileU T;
     T.init(a, t);
     T.run(a, L, nullptr, prof, PlainPos{ant}, r0, f0, nbeg, nend);
     store_tile(T, a, out, accumulate);
@@ -248,13 +247,6 @@ template <int TY, int PX, bool XL = false, int CAP = kBpCap>
 void launch_mixed_t(const BpArgs &a, int grid, const float2 *prof, const double *ant,
                     const double *r0, const double *f0, float2 *img, hipStream_t s) {
     hipLaunchKernelGGL((bp_mixed<TY, PX, XL, CAP>), dim3(grid), dim3(kBpThreads), 0, s, a, prof, ant,
-                       r0, f0, img);
-}
-
-template <int TL, int PX, bool XL>
-void launch_mixed_u(const BpArgs &a, int grid, const float2 *prof, const double *ant,
-                    const double *r0, const double *f0, float2 *img, hipStream_t s) {
-    hipLaunchKernelGGL((bp_mixed_u<TL, PX, XL>), dim3(grid), dim3(kBpThreads), 0, s, a, prof, ant,
                        r0, f0, img);
 }
 
@@ -577,7 +569,7 @@ int launch_mixed_shape(sarf_ctx *ctx, const sarf_bp_desc *d, int tile, int split
         case 15:
             if (for_gradient && five) launch_mixed_t<256, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, o, s);
             else if (for_gradient || !a.narrow) launch_mixed_t<256, 8, true>(a, grid, p, ant, r0, f0, o, s);
-            else launch_mixed_u<256, 8, true>(a, grid, p, ant, r0, f0, o, s);
+            else hipLaunchKernelGGL(bp_mixed_u, dim3(grid), dim3(kBpThreads), 0, s, a, p, ant, r0, f0, o);
             break;
         case 16:
             if (five) launch_mixed_t<128, 8, true, kBpCapX>(a, grid, p, ant, r0, f0, o, s);

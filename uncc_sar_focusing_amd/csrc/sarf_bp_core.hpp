@@ -563,13 +563,12 @@ struct BpTile {
 };
 
 // ---------------------------------------------------------------------------
-// BpTileU: tiles whose waves have one range of pixel-axis coordinates each (64
-// lanes or more along the lane axis), for image formation.  Same expansion of
-// the range as BpTile, kept in revolutions and regrouped around the middle of
-// the wave's PX pixels (P = Pc + d in pixel spacings, d = +-1/2, +-3/2, .., so
-// instruction literals):
+// BpTileU: tile 15 (256 lanes along x, 8 pixels per lane along y, so that all lanes
+// have the same pixel-axis coordinates) for image formation.  Same expansion of
+// the range as BpTile, kept in revolutions and regrouped around the tile's middle
+// row (P = d in pixel spacings, d = +-1/2, +-3/2, .., so instruction literals):
 //   phase(d) = by + d^2 kB + d kA,
-//   by = psi_c + rev(L, Pc), kA, kB its slope and half its curvature along P,
+//   by = psi_c + rev(L), kA, kB its slope and half its curvature along P,
 // per (pulse, lane) 11 instructions; then a pair of pixels +-d shares
 // by + d^2 kB, and the window position follows from the phase,
 //   p = phase * bins_per_revolution + bx,
@@ -595,9 +594,8 @@ struct BpTile {
 enum : int { kPulseFast = 0, kPulseGated = 1, kPulseDirect = 2 };
 constexpr int kBpWavesU = 5;  // waves per SIMD (workgroups per CU)
 
-template <int CH>
 struct BpLdsU {
-    static_assert(CH <= 64, "one wave stages a chunk");
+    static constexpr int CH = 64;  // pulses per chunk: one wave stages them
     float4 win[kBpCapX];
     // (k: revolutions per metre; w: pixel spacing along the pixel axis)
     float4 qA[CH];  // -k u_l, k c2l, k c3l, psi_c
@@ -609,44 +607,33 @@ struct BpLdsU {
     int nc, tot, fast;  // pulses staged, window bins staged, all of them kPulseFast
 };
 
-template <int TL_, int PX, bool XL>
 struct BpTileU {
-    static constexpr int TL = TL_;
-    static constexpr int GX = kBpThreads / TL;
-    static constexpr int NP = GX * PX;
-    static constexpr int kPx = PX;
-    static constexpr int TX = XL ? TL : NP;
-    static constexpr int TYE = XL ? NP : TL;
-    static constexpr int CH = TL == 256 ? 64 : kBpChunk;
-    static_assert(TL % 64 == 0 && PX % 2 == 0, "one range of pixel coordinates per wave");
-    using Lds = BpLdsU<CH>;
+    static constexpr int TX = kBpThreads, PX = 8;  // lanes along x, pixels per lane along y
+    static constexpr int kPx = PX, CH = BpLdsU::CH;
+    using Lds = BpLdsU;
     static_assert(kBpCapX * 16 <= 0x8000, "bin_bytes");
     static constexpr int kFx = 4;  // no per-column terms (BpTile's interface)
-    int ix0, iy0, ly, gx;
+    int ix0, iy0;
     double pcx, pcy, hx, hy;
     float ql;  // lane coordinate, tile-centred
-    float Pc;  // middle of the wave's pixels in pixel spacings (uniform)
     float accr[PX], acci[PX];
 
     __device__ __forceinline__ void init(const BpArgs &a, int t) {
         const int ty = t / a.tiles_x, tx = t - ty * a.tiles_x;
         ix0 = tx * TX;
-        iy0 = ty * TYE;
+        iy0 = ty * PX;
         pcx = a.left + (ix0 + 0.5 * (TX - 1)) * a.dx;
-        pcy = a.bottom + (iy0 + 0.5 * (TYE - 1)) * a.dy;
+        pcy = a.bottom + (iy0 + 0.5 * (PX - 1)) * a.dy;
         hx = 0.5 * (TX - 1) * a.dx;
-        hy = 0.5 * (TYE - 1) * a.dy;
-        ly = threadIdx.x % TL;
-        gx = __builtin_amdgcn_readfirstlane(threadIdx.x / TL);
-        ql = (float)((ly - 0.5 * (TL - 1)) * (XL ? a.dx : a.dy));
-        Pc = (float)(gx * PX) + 0.5f * (PX - NP);
+        hy = 0.5 * (PX - 1) * a.dy;
+        ql = (float)(((int)threadIdx.x - 0.5 * (TX - 1)) * a.dx);
 #pragma unroll
         for (int j = 0; j < PX; j++) accr[j] = acci[j] = 0.f;
     }
 
     __device__ __forceinline__ bool pixel(int j, int &x, int &y, const BpArgs &a) const {
-        x = XL ? ix0 + ly : ix0 + gx * PX + j;
-        y = XL ? iy0 + gx * PX + j : iy0 + ly;
+        x = ix0 + (int)threadIdx.x;
+        y = iy0 + j;
         return x < a.Nx && y < a.Ny;
     }
 
@@ -678,11 +665,11 @@ struct BpTileU {
                 double psi = kap * dRc;
                 psi -= rint(psi);
                 const double ah = ux * iR, bh = uy * iR, g0 = 0.5 * iR, g1 = 0.5 * iR * iR;
-                const double up = XL ? bh : ah, ul = XL ? ah : bh;
+                const double up = bh, ul = ah;
                 const double mp = 1.0 - up * up, ml = 1.0 - ul * ul;
                 L.qA[tid] = make_float4((float)(-kap * ul), (float)(kap * g0 * ml),
                                         (float)(kap * g1 * ul * ml), (float)psi);
-                const double w = XL ? a.dy : a.dx, kw = kap * w;
+                const double w = a.dy, kw = kap * w;
                 L.qB[tid] = make_float4((float)(-kw * up), (float)(-2.0 * kw * up * ul * g0),
                                         (float)(kw * g1 * up * (1.0 - 3.0 * ul * ul)),
                                         (float)(kw * w * g0 * mp));
@@ -695,8 +682,7 @@ struct BpTileU {
                 // half extent along the pixel axis; the cubic term there in
                 // revolutions, and a carrier so low that the phase cannot
                 // carry the position
-                const double hp = XL ? hy : hx;
-                if (!(wd <= kBpCapX) || !(fabs(kap) * g1 * hp * hp * hp <= 1e-6) ||
+                if (!(wd <= kBpCapX) || !(fabs(kap) * g1 * hy * hy * hy <= 1e-6) ||
                     !(fabsf(C.y) <= 1e4f))
                     mode = kPulseDirect;
                 else
@@ -733,12 +719,8 @@ struct BpTileU {
         const float4 B = L.qB[c];
         const float4 C = L.qC[c];
         const float kB = fmaf(ql, C.x, B.w);
-        float kA = fmaf(ql, fmaf(ql, B.z, B.y), B.x);
-        float rev = ql * fmaf(ql, fmaf(ql, A.z, A.y), A.x);
-        if constexpr (GX > 1) {
-            rev = fmaf(Pc, fmaf(Pc, kB, kA), rev);
-            kA = fmaf(2.f * Pc, kB, kA);
-        }
+        const float kA = fmaf(ql, fmaf(ql, B.z, B.y), B.x);
+        const float rev = ql * fmaf(ql, fmaf(ql, A.z, A.y), A.x);
         const float by = __builtin_amdgcn_fractf(A.w + rev);
         // window position (less kBinShift) at phase 0 of the reduced phase
         const float bx = fmaf(C.y, rev - by, C.z);
@@ -782,15 +764,15 @@ struct BpTileU {
         const float4 A = L.pA[c];
         const int start = L.pI[c].x;
         const float kap = L.kap[c], psi = L.qA[c].w, pos = L.qC[c].z + kBinShift;
-        const float ul = XL ? A.x : A.y, up = XL ? A.y : A.x;
+        const float ul = A.x, up = A.y;
         const float glo = (float)(-start), ghi = (float)(a.Nfft - 1 - start);
         // opaque, so that this path's per-pixel constants are not held in
         // registers through the others
-        float dp = (float)(XL ? a.dy : a.dx), mid = Pc;
-        __asm__ volatile("" : "+v"(dp), "+v"(mid));
+        float dp = (float)a.dy;
+        __asm__ volatile("" : "+v"(dp));
 #pragma unroll
         for (int j = 0; j < PX; j++) {
-            const float P = (mid + (j - 0.5f * (PX - 1))) * dp;
+            const float P = (j - 0.5f * (PX - 1)) * dp;
             const float s = fmaf(up, P, ul * ql);
             const float t = fmaf(-s, s, fmaf(P, P, ql * ql));
             const float dl = fmaf(t, fmaf(s, A.w, A.z), -s);

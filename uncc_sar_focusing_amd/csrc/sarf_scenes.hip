@@ -39,7 +39,7 @@ struct SceneDev {
 // the ones sarf_backproject runs.  Four workgroups per CU: with five, the
 // engines behind a call spilled in their loops (16 scenes 5.5 -> 6.1 ms).
 constexpr int kMixedIds[3] = {15, 16, 13};
-using MixedT0 = BpTileU<256, 8, true>;
+using MixedT0 = BpTileU;
 using MixedT1 = BpTile<128, 8, true>;
 using MixedT2 = BpTile<64, 8, true>;
 using MixedT3 = BpTile<256, 8, true>;
