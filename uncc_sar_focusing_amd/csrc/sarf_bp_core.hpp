@@ -576,7 +576,9 @@ struct BpTile {
 // BpTile takes 4 and two LDS reads.  by is reduced to one revolution first,
 // which leaves the phase a few revolutions at most: its rounding (the
 // error of the image) is no larger than before.
-// Pulses whose window or phase needs it take the gated form of the same.  The
+// A carrier of few revolutions per bin would magnify that rounding in p
+// (kBpPhaseBins); its pulses form p by itself, 3.5 FMA for both.  Pulses whose
+// window or phase needs it take the gated form of that.  The
 // direct expansion over the profile in memory remains for pulses whose window
 // does not fit in LDS, that are so near that the cubic term along the pixel
 // axis (left out here) would show, or that have no carrier to speak of.
@@ -591,8 +593,14 @@ struct BpTile {
 // 8 pixels, 128 VGPRs, four waves) 6.29.  Only tile 15: tiles 16 and 13 keep
 // the rounding of BpTile, which is most of what their images are off by.
 // ---------------------------------------------------------------------------
-enum : int { kPulseFast = 0, kPulseGated = 1, kPulseDirect = 2 };
+enum : int { kPulseFast = 0, kPulseCoarse = 1, kPulseGated = 2, kPulseDirect = 3 };
 constexpr int kBpWavesU = 5;  // waves per SIMD (workgroups per CU)
+// Most bins per revolution for which the position is taken from the phase: the
+// phase's rounding, an ulp of a revolution or two (1.2e-7 to 2.4e-7), is then 2e-6 of
+// a bin, an ulp of a position being 8e-6 to 1.2e-4.  rel-L2 of white samples, 300 x
+// 200 at 0.05 m: 5.3 bins per revolution 1.05e-6 either way; 17.5 from the phase
+// 1.23e-6, by itself 0.99e-6; 5250 1.9e-4 and 0.97e-6.
+constexpr float kBpPhaseBins = 8.f;
 
 struct BpLdsU {
     static constexpr int CH = 64;  // pulses per chunk: one wave stages them
@@ -603,7 +611,7 @@ struct BpLdsU {
     float4 qC[CH];  // k w^2 e3, bins per revolution, pos_c - kBinShift, kBinMagic + LDS offset (bins)
     int4 pI[CH];    // start bin, LDS offset, W, kPulse*
     float4 pA[CH];  // direct form: uh_x, uh_y, g0, g1
-    float kap[CH];
+    float4 pB[CH];  // slopes of the window position -b u_l, -b w u_p (b: bins per metre); k
     int nc, tot, fast;  // pulses staged, window bins staged, all of them kPulseFast
 };
 
@@ -676,9 +684,9 @@ struct BpTileU {
                 C = make_float4((float)(kw * w * g1 * ul * (1.0 - 3.0 * up * up)),
                                 (float)(a.binv / kap), (float)(posg - st - kBinShift), 0.f);
                 L.pA[tid] = make_float4((float)ah, (float)bh, (float)g0, (float)g1);
-                L.kap[tid] = (float)kap;
+                L.pB[tid] = make_float4((float)(-a.binv * ul), (float)(-a.binv * w * up), (float)kap, 0.f);
                 const bool inside = st >= 0.0 && st + wd <= a.Nfft && fabs(kap) * ext <= 250.0;
-                mode = inside ? kPulseFast : kPulseGated;
+                mode = !inside ? kPulseGated : fabsf(C.y) <= kBpPhaseBins ? kPulseFast : kPulseCoarse;
                 // half extent along the pixel axis; the cubic term there in
                 // revolutions, and a carrier so low that the phase cannot
                 // carry the position
@@ -712,9 +720,10 @@ struct BpTileU {
         __syncthreads();
     }
 
-    // One staged pulse, kPulseFast or kPulseGated.
-    template <bool GATED>
+    // One staged pulse, kPulseFast, kPulseCoarse or kPulseGated.
+    template <int MODE>
     __device__ __forceinline__ void pulse(const BpArgs &a, const Lds &L, int c) {
+        constexpr bool GATED = MODE == kPulseGated;
         const float4 A = L.qA[c];
         const float4 B = L.qB[c];
         const float4 C = L.qC[c];
@@ -722,8 +731,17 @@ struct BpTileU {
         const float kA = fmaf(ql, fmaf(ql, B.z, B.y), B.x);
         const float rev = ql * fmaf(ql, fmaf(ql, A.z, A.y), A.x);
         const float by = __builtin_amdgcn_fractf(A.w + rev);
-        // window position (less kBinShift) at phase 0 of the reduced phase
-        const float bx = fmaf(C.y, rev - by, C.z);
+        // window position (less kBinShift): at phase 0 of the reduced phase, or by
+        // itself at the middle row, with its slope and half its curvature
+        float bx, pA = 0.f, pB = 0.f;
+        if constexpr (MODE == kPulseFast) {
+            bx = fmaf(C.y, rev - by, C.z);
+        } else {
+            const float4 b = L.pB[c];
+            bx = fmaf(ql, fmaf(C.y * ql, fmaf(ql, A.z, A.y), b.x), C.z);
+            pA = fmaf(C.y, ql * fmaf(ql, B.z, B.y), b.y);
+            pB = C.y * kB;
+        }
         const char *win = (const char *)L.win;
         float glo = 0.f, ghi = 0.f, wmax = 0.f;
         if constexpr (GATED) {
@@ -740,8 +758,8 @@ struct BpTileU {
         for (int j = 0; j < PX; j++) {
             const float d = j - 0.5f * (PX - 1);
             ph[j] = fmaf(d, kA, fmaf(d * d, kB, by));
-            p[j] = fmaf(ph[j], C.y, bx);
-            // fast: the window has a bin of margin on each side, 1 <= p <= W - 2
+            p[j] = MODE == kPulseFast ? fmaf(ph[j], C.y, bx) : fmaf(d, fmaf(d, pB, pA), bx);
+            // not gated: the window has a bin of margin on each side, 1 <= p <= W - 2
             w[j] = *(const float4 *)(win + bin_bytes(GATED ? __builtin_amdgcn_fmed3f(p[j], 0.f, wmax) : p[j], C.w));
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -763,7 +781,7 @@ struct BpTileU {
                                                  const float2 *__restrict__ row) {
         const float4 A = L.pA[c];
         const int start = L.pI[c].x;
-        const float kap = L.kap[c], psi = L.qA[c].w, pos = L.qC[c].z + kBinShift;
+        const float kap = L.pB[c].z, psi = L.qA[c].w, pos = L.qC[c].z + kBinShift;
         const float ul = A.x, up = A.y;
         const float glo = (float)(-start), ghi = (float)(a.Nfft - 1 - start);
         // opaque, so that this path's per-pixel constants are not held in
@@ -802,12 +820,13 @@ struct BpTileU {
             stage(a, L, prof, pos, r0, f0, n0, min(CH, nend - n0));
             const int nc = L.nc;
             if (__builtin_amdgcn_readfirstlane(L.fast)) {
-                for (int c = 0; c < nc; c++) pulse<false>(a, L, c);
+                for (int c = 0; c < nc; c++) pulse<kPulseFast>(a, L, c);
             } else {
                 for (int c = 0; c < nc; c++) {
                     const int mode = __builtin_amdgcn_readfirstlane(L.pI[c].w);
-                    if (mode == kPulseFast) pulse<false>(a, L, c);
-                    else if (mode == kPulseGated) pulse<true>(a, L, c);
+                    if (mode == kPulseFast) pulse<kPulseFast>(a, L, c);
+                    else if (mode == kPulseCoarse) pulse<kPulseCoarse>(a, L, c);
+                    else if (mode == kPulseGated) pulse<kPulseGated>(a, L, c);
                     else pulse_direct(a, L, c, prof + (size_t)(n0 + c) * a.Nfft);
                 }
             }
