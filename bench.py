@@ -483,7 +483,8 @@ def main() -> int:
         "frac": round(achieved / PEAK_FP32_TFLOPS, 4),
         "traffic": traffic,
         "traffic_source": traffic_src,
-        "kernel": "bp_mixed",
+        # tile 15, unless its windows are wider than the kernel's
+        "kernel": "bp_mixed_u" if (tune or {}).get("tile") == 15 else "bp_mixed",
         "trans_frac": round(TRANS_PER_PP * pp / (t_bp * 1e-3) / 1e12 / PEAK_TRANS_TOPS, 4),
         "nonpacked_fp32_measured": MEASURED_NONPACKED_TFLOPS,
         "frac_of_nonpacked": round(achieved / MEASURED_NONPACKED_TFLOPS, 4),

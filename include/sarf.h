@@ -79,10 +79,12 @@ const char *sarf_last_error(void);
  * captured: a caller that captures work of one context on several streams
  * orders them itself.  Scratch that has to grow is kept, not freed, until
  * sarf_ctx_trim or sarf_ctx_destroy, so work enqueued earlier (or a captured
- * graph) never refers to freed memory.  Tables a transform length needs
- * (twiddles, Bluestein chirps and their spectra) are built on its first use
- * in the context, on the host with a synchronous upload, and kept until
- * sarf_ctx_destroy: capture a call into a HIP graph after one eager call
+ * graph) never refers to freed memory.  Tables that sizes need (twiddles of a
+ * transform length; Bluestein chirps and their spectra of an Nfft and, up to
+ * 8192, the power of two that Nfft + K - 1 rounds up to; matched-filter weights
+ * of a K) are built on their first use in the context, on the host with a
+ * synchronous upload, and kept until sarf_ctx_destroy, and scratch grows on
+ * first use: capture a call into a HIP graph after one eager call
  * with the same sizes. */
 int sarf_ctx_create(int device, sarf_ctx **out);
 int sarf_ctx_destroy(sarf_ctx *ctx);
@@ -169,8 +171,8 @@ typedef struct {
                        batches and the gradient take 1..5 and 11..16 */
     int pulse_split;/* 0 = automatic; n >= 1: pulses in n contiguous groups summed
                        in group order -- n even groups, each a partial image, or,
-                       when the image's tiles fill two rounds of resident
-                       workgroups, one head group of the first 7/8 of the pulses
+                       when the image's tiles number at least 8 per CU for most
+                       tile ids, one head group of the first 7/8 of the pulses
                        written into img and n - 1 tail groups as partial images */
     double los_x, los_y; /* optional hint: horizontal components of the unit line
                             of sight from the image centre to the aperture centre;
@@ -407,10 +409,13 @@ int sarf_fit_quadratic(const float *values, int n, int skip, float *coeffs /* 3 
 /* Adjoint backprojection: grad[n] = dE/da_n (FP64, Np x 3), the gradient    */
 /* of the image entropy with respect to each antenna phase centre (R0 held   */
 /* fixed), given the forward image img = sarf_backproject(...) of the same   */
-/* inputs and ent = sarf_image_entropy(img).  Interpolated profile values    */
-/* are recomputed, nothing per pixel-pulse is stored.  No counterpart in the */
-/* reference; it makes the grid search of src/autofocus/autofocus_gpu.cu     */
-/* a gradient search.                                                       */
+/* inputs and ent = sarf_image_entropy(img).  With SARF_BP_FOR_GRADIENT the  */
+/* image is rounded as the values recomputed here are; without, the gradient */
+/* is as close to the FP64 one (512^2, 1024 pulses: rel-L2 3.3e-6 with the   */
+/* flag, 2.7e-6 without; 300^2, 400 pulses: 6.6e-6 both).  Interpolated      */
+/* profile values are recomputed, nothing per pixel-pulse is stored.  No     */
+/* counterpart in the reference; it makes the grid search of                 */
+/* src/autofocus/autofocus_gpu.cu a gradient search.                        */
 /* ------------------------------------------------------------------------ */
 int sarf_bp_entropy_grad(sarf_ctx *ctx, const sarf_bp_desc *desc,
                          const void *prof,    /* device float2 Nfft x Np */

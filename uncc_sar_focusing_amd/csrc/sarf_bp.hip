@@ -362,8 +362,8 @@ int bp_tile_shape(int id, int *tx, int *ty) {
     return 0;
 }
 
-// Waves per SIMD the tile's kernel is built for (= resident workgroups per
-// CU: 256-thread workgroups, 4 SIMDs); 1 for an unknown id.
+// Waves per SIMD of the tile's kernel with the 2048-bin windows (= its resident
+// workgroups per CU: 256-thread workgroups, 4 SIMDs); 1 for an unknown id.
 int tile_waves_per_eu(int tile) {
     for (const TileShape &t : kTiles)
         if (t.id == tile) return bp_waves_per_eu_rt(t.tl, t.px, t.xl != 0);
@@ -450,8 +450,10 @@ std::array<uint64_t, 8> tune_key(const sarf_bp_desc *d) { return tune_key(tune_g
 
 // Pulse splits.  A tile's pulses are split into groups, each a workgroup of
 // its own writing a partial image, summed in order afterwards.  Two rules:
-// * head + tail, when the tiles alone fill at least two rounds of resident
-//   workgroups: one head group of the first 7/8 of the pulses per tile
+// * head + tail, when there are at least twice as many tiles as workgroups of the
+//   tile's kernel with the 2048-bin windows are resident (8 tiles per CU for most;
+//   the five-wave kernels hold 10, and 2048 tiles of tile 15 measured best so among
+//   79 shapes too): one head group of the first 7/8 of the pulses per tile
 //   writes the image directly, and the last 1/8 is spread over splits - 1
 //   short groups that the split-major launch order runs last, filling in as
 //   CUs free up (default 3 splits).  Measured on MI355X at 2048^2 x 4096
